@@ -232,17 +232,23 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
 // y[M,N] = x[M,K] . w[N,K]^T (+ bias[N]) on f32 tensors (linear()'s TensorF32 arm)
 tlhip_status launch_linear_f32(hipStream_t s, const float* x, const float* w, const float* bias, float* y, int M, int N,
                                int K);
-bool gemm_skinny_ok(int M, int N, int K, int wt);   // the skinny M <= 64 GEMM takes the shape (and EPI_QKV_ROPE)
-// Split-K partials (fp32) of any count gemm_splits picks stay within
-// GEMM_SPLIT_PARTIALS_MAX bytes: M > 64 keeps tiles x slices <= GEMM_SPLIT_TILE_CAP
-// tiles of 128 x 128 (20 MiB); the skinny GEMM (5 <= M <= 64) splits at most
-// SK_MAX_TILES_SPLIT tiles (N <= 8192 at 64 rows) into 8 slices (16 MiB); the
-// other M <= 64 shapes keep tiles x slices <= 512 tiles of 64 x 64 (8 MiB).
-// kernels_gemm.hip ties these figures to its tile constants by static_assert.
-constexpr int GEMM_SPLIT_TILE_CAP = 320;
-constexpr size_t GEMM_SPLIT_PARTIALS_MAX = (size_t)GEMM_SPLIT_TILE_CAP * 128 * 128 * sizeof(float);
-int gemm_splits(int M, int N, int K, int wt);   // split-K slices launch_gemm uses when given a workspace
-                                                // (wt < 0: any weight type, the largest count)
+bool gemm_rope_ok(int M, int N, int K, int wt);   // the MFMA GEMM takes the shape with EPI_QKV_ROPE
+// the tiled GEMM's tile shape and K split (kernels_gemm_tile.hip)
+struct TilePlan {
+    int shape = 0, splits = 1;
+    size_t ws_bytes = 0;   // fp32 partials of the split (rows rounded up to 8 columns)
+    double us = 0.0;       // the cost model's estimate
+};
+TilePlan tile_plan(int M, int N, int K, int wt);
+tlhip_status launch_gemm_tile(hipStream_t s, int wt, const GemvArgs& a, int epi, int ldy, const TilePlan& pl);
+// Split-K partials (fp32) stay within GEMM_SPLIT_PARTIALS_MAX bytes: the tiled
+// GEMM's plan keeps its slices' partials to it, and the skinny GEMM (5 <= M <=
+// 64) splits at most SK_MAX_TILES_SPLIT tiles (N <= 8192 at 64 rows) into 8
+// slices (16 MiB).
+constexpr size_t GEMM_SPLIT_PARTIALS_MAX = (size_t)20 << 20;
+// bytes of split-K partials launch_gemm uses when given them as a workspace
+// (0: no split; wt < 0: the most any weight type uses)
+size_t gemm_ws_bytes(int M, int N, int K, int wt);
 uint16_t f32_to_f16(float f);            // host RNE rounding (F32 GGUF tensors)
 // Rows 0..src_rows-1 of a GGUF block stream [src_rows, K] go to rows
 // dst_row0 + r * dst_step of a packed tensor of dst_rows rows (to_gguf = 1:

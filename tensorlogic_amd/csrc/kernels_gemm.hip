@@ -1,26 +1,22 @@
 // kernels_gemm.hip -- dequant-GEMM for prefill (M > 4) on MFMA, gfx950.
 //
-// y[M, N] = x[M, K] . W[N, K]^T, W packed Q4_0 / Q8_0 or f16.  Each K step
-// stages an activation tile and a weight tile in LDS; the weight tile is
-// dequantised while it is written to LDS (RNE_f16((q-8)*d) / RNE_f16(q*d)
-// with v_pk_mul_f16, the exact values of gguf.rs:22-112), then the matrix
-// cores accumulate in fp32 as the reference's tiled matmul does
-// (unified.metal:4291-4348): v_mfma_f32_32x32x16_f16 in gemm2_kernel and
-// gemm_lds_kernel, v_mfma_f32_16x16x32_f16 in gemm_skinny_kernel, and
-// v_mfma_f32_32x32x8_f16 in the K % 64 != 0 fallback gemm_kernel.  Output
-// f16 with the same epilogues as the GEMV (bias, residual add, SwiGLU on
-// interleaved gate/up rows).
+// y[M, N] = x[M, K] . W[N, K]^T, W packed Q4_0 / Q8_0 or f16: activation and
+// weight tiles staged in LDS, weights dequantised to RNE_f16((q-8)*d) /
+// RNE_f16(q*d) (the exact values of gguf.rs:22-112), fp32 accumulation on the
+// matrix cores as the reference's tiled matmul does (unified.metal:
+// 4291-4348), output f16 with the same epilogues as the GEMV (bias, residual
+// add, SwiGLU on interleaved gate/up rows, QKV + RoPE + cache).
 //
-// Four kernels: gemm_kernel (K % 64 != 0; 64 x 64 x 32 tiles),
-// gemm_skinny_kernel (M <= 64: a ring of LDS stages per wave filled by
-// direct global->LDS loads, split over K with a fence-free exchange),
-// gemm2_kernel (register-staged, two LDS buffers, where the skinny plan does
-// not apply) and gemm_lds_kernel (M > 64: 128 x 128 tiles, three or four
-// LDS stages filled by direct global->LDS loads).
+// gemm_tile_kernel (gemm_tile.hpp, kernels_gemm_tile.hip) takes every K that
+// is a multiple of 32; gemm_skinny_kernel (below) the M <= 64 shapes where it
+// is the faster one: a ring of LDS stages per wave filled by direct
+// global->LDS loads, split over K with a fence-free exchange.  gemm_kernel
+// (64 x 64 x 32 tiles) covers rows too long for the tiled kernel's buffer
+// ranges, gemm_naive_kernel f16 weights whose K is no multiple of 32.  Here
+// too: linear() on f32 tensors.
 #include <type_traits>
 
-#include "device_common.hpp"
-#include "internal.hpp"
+#include "gemm_tile.hpp"
 
 namespace tlhip {
 
@@ -130,275 +126,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Pipelined MFMA GEMM (K % 64 == 0): tile BM x BN x 64 (two quant blocks per
-// K step), 256 threads as WM x WN waves, each wave owning (BM/WM) x (BN/WN)
-// of C in 32 x 32 v_mfma_f32_32x32x16_f16 tiles.  Two LDS buffers: the
-// global loads of step k+1 are issued into registers before the MFMAs of
-// step k, then dequantised into the other buffer (one barrier per step).
-// With split-K (gridDim.z > 1) each z-slice writes fp32 partials of a
-// contiguous K range and gemm_reduce_kernel sums the slices in z order and
-// applies the epilogue.
-// ---------------------------------------------------------------------------
-constexpr int G2_BK = 64, G2_PAD = 8;
-
-template <int WT, int BN>
-struct G2W {   // per-thread global weight registers of one K step
-    static constexpr int NV = WT == TLHIP_F16 ? BN * 8 / 256 : (WT == TLHIP_Q8_0 ? BN * 4 / 256 : (BN * 2 + 255) / 256);
-};
-
-template <int WT, int BM, int BN>
-__device__ __forceinline__ void g2_load(const GemmParams& p, int m0, int n0, int kt, int tid,
-                                        u4 (&xr)[BM * 8 / 256], u4 (&wr)[G2W<WT, BN>::NV], uint16_t& dsc) {
-    constexpr int XV = BM * 8 / 256;          // 16-byte chunks of x per thread
-    constexpr int TPR = 8 / XV;               // threads per x row
-    const int nbr = p.K >> 5;
-    {
-        const int r = tid / TPR, c0 = (tid % TPR) * XV;
-        const int m = m0 + r;
-#pragma unroll
-        for (int v = 0; v < XV; v++)
-            xr[v] = m < p.M ? *(const u4*)(p.x + (size_t)m * p.K + (size_t)kt * G2_BK + 8 * (c0 + v)) : u4{0u, 0u, 0u, 0u};
-    }
-    if (WT == TLHIP_Q4_0) {
-        // (row, block) pairs: tid -> row tid/2, block tid%2; 16 payload bytes + scale
-        if (tid < BN * 2) {
-            const int n = min(n0 + (tid >> 1), p.N - 1), b = 2 * kt + (tid & 1);
-            wr[0] = *(const u4*)(p.wq + (size_t)n * (p.K / 2) + (size_t)b * 16);
-            dsc = p.wd[(size_t)n * nbr + b];
-        }
-    } else if (WT == TLHIP_Q8_0) {
-        // tid -> row tid/4, block (tid/2)%2, half tid%2: 16 int8 + scale
-        const int n = min(n0 + (tid >> 2), p.N - 1), b = 2 * kt + ((tid >> 1) & 1);
-        wr[0] = *(const u4*)(p.wq + (size_t)n * p.K + (size_t)b * 32 + 16 * (tid & 1));
-        dsc = p.wd[(size_t)n * nbr + b];
-    } else {
-        constexpr int NV = G2W<WT, BN>::NV;
-        const int r = tid / (8 / NV), c0 = (tid % (8 / NV)) * NV;
-        const int n = min(n0 + r, p.N - 1);
-#pragma unroll
-        for (int v = 0; v < NV; v++)
-            wr[v] = *(const u4*)((const uint16_t*)p.wq + (size_t)n * p.K + (size_t)kt * G2_BK + 8 * (c0 + v));
-    }
-}
-
-template <int WT, int BM, int BN>
-__device__ __forceinline__ void g2_store(int tid, const u4 (&xr)[BM * 8 / 256], const u4 (&wr)[G2W<WT, BN>::NV],
-                                         uint16_t dsc, uint16_t (*As)[G2_BK + G2_PAD],
-                                         uint16_t (*Bs)[G2_BK + G2_PAD]) {
-    constexpr int XV = BM * 8 / 256;
-    constexpr int TPR = 8 / XV;
-    {
-        const int r = tid / TPR, c0 = (tid % TPR) * XV;
-#pragma unroll
-        for (int v = 0; v < XV; v++) *(u4*)&As[r][8 * (c0 + v)] = xr[v];
-    }
-    if (WT == TLHIP_Q4_0) {
-        if (tid < BN * 2) {
-            const int r = tid >> 1, c = 32 * (tid & 1);
-            const h16 dh = __builtin_bit_cast(h16, dsc);
-            const h2 dd = {dh, dh};
-            uint32_t lo[8], hi[8];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                h2 q[4];
-                q4_unpack(wr[0][t], dd, q);
-                lo[2 * t] = pack_lo(as_u32(q[0]), as_u32(q[1]));
-                lo[2 * t + 1] = pack_hi(as_u32(q[0]), as_u32(q[1]));
-                hi[2 * t] = pack_lo(as_u32(q[2]), as_u32(q[3]));
-                hi[2 * t + 1] = pack_hi(as_u32(q[2]), as_u32(q[3]));
-            }
-            *(u4*)&Bs[r][c + 0] = u4{lo[0], lo[1], lo[2], lo[3]};
-            *(u4*)&Bs[r][c + 8] = u4{lo[4], lo[5], lo[6], lo[7]};
-            *(u4*)&Bs[r][c + 16] = u4{hi[0], hi[1], hi[2], hi[3]};
-            *(u4*)&Bs[r][c + 24] = u4{hi[4], hi[5], hi[6], hi[7]};
-        }
-    } else if (WT == TLHIP_Q8_0) {
-        const int r = tid >> 2, c = 32 * ((tid >> 1) & 1) + 16 * (tid & 1);
-        const h16 dh = __builtin_bit_cast(h16, dsc);
-        const h2 dd = {dh, dh};
-        uint32_t o[8];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            h2 q[2];
-            q8_unpack(wr[0][t], dd, q);
-            o[2 * t] = pack_lo(as_u32(q[0]), as_u32(q[1]));
-            o[2 * t + 1] = pack_hi(as_u32(q[0]), as_u32(q[1]));
-        }
-        *(u4*)&Bs[r][c + 0] = u4{o[0], o[1], o[2], o[3]};
-        *(u4*)&Bs[r][c + 8] = u4{o[4], o[5], o[6], o[7]};
-    } else {
-        constexpr int NV = G2W<WT, BN>::NV;
-        const int r = tid / (8 / NV), c0 = (tid % (8 / NV)) * NV;
-#pragma unroll
-        for (int v = 0; v < NV; v++) *(u4*)&Bs[r][8 * (c0 + v)] = wr[v];
-    }
-}
-
-__device__ __forceinline__ void gemm_store_one(const GemmParams& p, int m, int n, float v) {
-    if (p.epi == EPI_SWIGLU_PAIR) {
-        const float up = __shfl_down(v, 1, 64);
-        if (m < p.M && n + 1 < p.N && (n & 1) == 0) p.y[(size_t)m * p.ldy + n / 2] = swiglu_h(f2h(v), f2h(up));
-    } else if (m < p.M && n < p.N) {
-        p.y[(size_t)m * p.ldy + n] = epilogue_h(p.epi, v, p.bias, p.resid, (size_t)m * p.N + n, n);
-    }
-}
-
-template <int WT, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256) void gemm2_kernel(GemmParams p, float* __restrict__ part) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM][G2_BK + G2_PAD];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN][G2_BK + G2_PAD];
-    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
-    constexpr int XV = BM * 8 / 256;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int nkt = p.K / G2_BK;
-    const int kt0 = (int)((int64_t)nkt * blockIdx.z / gridDim.z), kt1 = (int)((int64_t)nkt * (blockIdx.z + 1) / gridDim.z);
-    f16v acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f16v{0};
-
-    u4 xr[XV], wr[G2W<WT, BN>::NV];
-    uint16_t dsc = 0;
-    if (kt0 < kt1) {
-        g2_load<WT, BM, BN>(p, m0, n0, kt0, tid, xr, wr, dsc);
-        g2_store<WT, BM, BN>(tid, xr, wr, dsc, As[0], Bs[0]);
-    }
-    __syncthreads();
-    for (int kt = kt0; kt < kt1; kt++) {
-        const int buf = (kt - kt0) & 1;
-        const bool more = kt + 1 < kt1;
-        if (more) g2_load<WT, BM, BN>(p, m0, n0, kt + 1, tid, xr, wr, dsc);
-#pragma unroll
-        for (int ks = 0; ks < G2_BK; ks += 16) {
-            const int kk = ks + 8 * (lane >> 5);
-            h8 a[TM], b[TN];
-#pragma unroll
-            for (int i = 0; i < TM; i++) a[i] = *(const h8*)&As[buf][wm * (BM / WM) + 32 * i + (lane & 31)][kk];
-#pragma unroll
-            for (int j = 0; j < TN; j++) b[j] = *(const h8*)&Bs[buf][wn * (BN / WN) + 32 * j + (lane & 31)][kk];
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) g2_store<WT, BM, BN>(tid, xr, wr, dsc, As[buf ^ 1], Bs[buf ^ 1]);
-        __syncthreads();
-    }
-
-    // C layout: col = lane%32 (weight row n), row = 8*(r/4) + 4*(lane/32) + r%4 (activation row m)
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn * (BN / WN) + 32 * j + (lane & 31);
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * (BM / WM) + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const float v = acc[i][j][r];
-                if (part) {
-                    if (m < p.M && n < p.N) part[((size_t)blockIdx.z * p.M + m) * p.N + n] = v;
-                } else {
-                    gemm_store_one(p, m, n, v);
-                }
-            }
-        }
-}
-
-// ---------------------------------------------------------------------------
-// Multi-stage MFMA dequant-GEMM (K % 64 == 0).  Workgroup tile BM x BN x 64,
-// 512 threads = 8 waves in a 2 (M) x 4 (N) grid, each wave (BM/2) x (BN/4) of
-// C in 32 x 32 v_mfma_f32_32x32x16_f16 tiles.  NS LDS stages are filled by
-// direct global->LDS loads (global_load_lds_dwordx4 / _dword, no VGPR
-// staging), so NS - 1 K steps are in flight while one is computed.  The LDS
-// keeps the GGUF payload as stored (Q4_0 nibbles, Q8_0 int8 or f16) plus the
-// block scales; each wave dequantises its B operand from LDS into registers
-// right before its MFMAs, with the same RNE_f16((q-8)*d) / RNE_f16(q*d) as
-// every other path.
-//
-// K order inside a 64-wide step: MFMA lane half h (lane / 32) carries the
-// elements 32h + 8t .. 32h + 8t + 7 at sub-step t = 0..3 (quant block h of
-// the step) for A and B alike, so every k is summed once in fp32.
-//
-// LDS rows are XOR-swizzled in 16-byte chunks so that the 32 rows a wave
-// reads at one chunk index fall in distinct banks: A / f16 B rows (128 B)
-// chunk c -> c ^ ((r >> 1) & 7); Q8_0 rows (64 B) c -> c ^ ((r >> 2) & 3); Q4_0 rows
-// (32 B) c -> c ^ ((r >> 3) & 1).  A direct load writes lane l's 16 (4) bytes
-// at LDS base + 16 l (4 l); each lane fetches the global chunk that the
-// swizzle puts in its slot.
-//
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup id mod
-// 8); the id -> tile map gives each XCD a contiguous run of tiles with the
-// M tiles of one N tile adjacent, so the BM-row tiles that share a weight
-// tile run on one XCD and read it through one L2.
-// ---------------------------------------------------------------------------
-
-template <int WT>
-struct GlRow {   // LDS bytes of one weight row per 64-wide K step
-    static constexpr int B = WT == TLHIP_F16 ? 128 : (WT == TLHIP_Q8_0 ? 64 : 32);
-};
-
-// direct loads of one LDS region of R bytes by 512 threads: 16-byte loads
-// when R is a multiple of 8 KB, else 4-byte loads (R multiple of 2 KB)
-template <int R>
-struct GlDma {
-    static constexpr int SZ = R % 8192 == 0 ? 16 : 4;
-    static constexpr int N = R / (512 * SZ);
-    static_assert(R % 2048 == 0, "region");
-};
-
-template <int WT, int BM, int BN, int NS>
-struct Gl {
-    static constexpr int A_BYTES = BM * 128;
-    static constexpr int B_BYTES = BN * GlRow<WT>::B;
-    static constexpr int S_BYTES = WT == TLHIP_F16 ? 0 : BN * 4;
-    static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;
-    static constexpr int VMC = GlDma<A_BYTES>::N + GlDma<B_BYTES>::N + (S_BYTES ? 1 : 0);
-    static_assert((NS - 2) * VMC < 64, "vmcnt range");
-    static_assert(BN / 8 <= 64, "scale rows per wave");
-};
-
-template <int N>
-__device__ __forceinline__ void gl_wait_vm() {   // s_waitcnt vmcnt(N), gfx9 encoding
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70 | 0xF00);
-}
-template <int VMC, int K>
-__device__ __forceinline__ void gl_wait_stage(int ahead) {   // wait until <= ahead stages outstanding
-    if constexpr (K == 0) {
-        gl_wait_vm<0>();
-    } else {
-        if (ahead >= K) gl_wait_vm<K * VMC>();
-        else gl_wait_stage<VMC, K - 1>(ahead);
-    }
-}
-
-template <int SZ>
-__device__ __forceinline__ void gl_dma(const void* g, uint8_t* lds) {
-    if constexpr (SZ == 16) __builtin_amdgcn_global_load_lds(g, (gl_lds_t)lds, 16, 0, 0);
-    else __builtin_amdgcn_global_load_lds(g, (gl_lds_t)lds, 4, 0, 0);
-}
-
-// Four payload bytes -> two f16 pairs in element order (e0,e1) (e2,e3).
-__device__ __forceinline__ void q8_pairs(uint32_t w, h2 dd, uint32_t& p01, uint32_t& p23) {
-    const h2 bias = {(h16)-1152.0f, (h16)-1152.0f};
-    const uint32_t v = w ^ 0x80808080u;
-    p01 = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)) + bias) * dd);
-    p23 = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)) + bias) * dd);
-}
-__device__ __forceinline__ void q4_pairs(uint32_t nib, h2 dd, uint32_t& p01, uint32_t& p23) {
-    const h2 bias = {(h16)-1032.0f, (h16)-1032.0f};
-    p01 = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u)) + bias) * dd);
-    p23 = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u)) + bias) * dd);
-}
-
-__device__ __forceinline__ int gl_tile(int id, int T) {   // XCD-contiguous tile order
-    const int x = id & 7, s = id >> 3, q = T >> 3, r = T & 7;
-    return x * q + min(x, r) + s;
-}
-
-// ---------------------------------------------------------------------------
 // Skinny dequant-GEMM (4 < M <= 64, K % 64 == 0) on v_mfma_f32_16x16x32_f16:
 // one launch, no workspace by default.  A workgroup reads its activation
 // rows and weight rows once; both enter the CU as whole 64-byte pieces,
@@ -442,7 +169,6 @@ __device__ __forceinline__ int gl_tile(int id, int T) {   // XCD-contiguous tile
 // output's summation order, and so its bits, unchanged.
 // ---------------------------------------------------------------------------
 constexpr int SK_LDS = 160 * 1024 - 1024;   // LDS the rings may take
-constexpr uint32_t SK_OOB = 0x80000000u;    // a buffer offset past every tensor
 constexpr int SK_MAX_SPLITS = 8;
 
 template <int WT, int MT, int NT, int KP>
@@ -819,7 +545,7 @@ __global__ __launch_bounds__(64 * KP) void gemm_skinny_kernel(GemmParams p) {
     }
 }
 
-bool gemm_skinny_ok(int M, int N, int K, int wt) {
+static bool gemm_skinny_ok(int M, int N, int K, int wt) {
     // byte offsets of the buffer loads are 32-bit, the padding offset
     // SK_OOB above every tensor
     const uint64_t wrow = wt == TLHIP_F16 ? 2ull * K : (wt == TLHIP_Q4_0 ? K / 2ull : (uint64_t)K);
@@ -843,6 +569,7 @@ bool gemm_skinny_ok(int M, int N, int K, int wt) {
 // nothing else fits; a split leaves each wave at least two 64-k steps.
 struct SkPlan {
     int mt = 1, nt = 2, kp = 4, mtiles = 1, splits = 1;
+    double us = 0.0;   // the model's estimate
 };
 static int sk_stage_bytes(int wt, int mt, int nt) {
     const int wrow = wt == TLHIP_F16 ? 128 : (wt == TLHIP_Q8_0 ? 64 : 32);
@@ -876,9 +603,51 @@ static SkPlan sk_plan(int M, int N, int K, int wt) {
                     }
                 }
             }
+        best.us = best_us;
         if (best_us < 1e30) break;
     }
     return best;
+}
+
+// Skinny or tiled for M <= 64, by the two cost models.  sk_plan ranks skinny
+// plans among themselves; against measured launches (154 shapes, M 5 - 64) its
+// estimate e is right for Q8_0, 1.2 e for Q4_0 and 3 + e / 2 for f16, and the
+// tiled kernel's is 1 us high for f16.  The margins are for weights that
+// come from HBM, where the skinny kernel's many small workgroups start sooner:
+// M = 46, Q4_0, in a 22-layer prompt pass, skinny / tiled: [2560 x 2048] 8.6 /
+// 10.3 us, [2048 x 2048] 7.5 / 9.8, [2048 x 5632] 10.6 / 11.9, [11264 x 2048]
+// 14.3 / 11.9.
+struct GemmPlan {
+    int M = -1, N = 0, K = 0, wt = 0;
+    bool skinny = false;
+    SkPlan sk;
+    TilePlan tile;
+    size_t ws_bytes = 0;   // split-K partials
+};
+
+// the tiled kernel's buffer ranges (128 rows of x) are below 2^31 bytes
+static bool tile_ok(int K) { return K % 32 == 0 && K <= (1 << 22); }
+
+// The plan of a shape, kept per thread for the shapes seen last (a model's
+// prompt pass asks for the same few over and over; evaluating both models
+// costs about a microsecond of host time).
+static const GemmPlan& gemm_plan(int M, int N, int K, int wt) {
+    static thread_local GemmPlan kept[64];
+    GemmPlan& p = kept[((uint32_t)M * 2654435761u ^ (uint32_t)N * 40503u ^ (uint32_t)K * 9176u ^ (uint32_t)wt) >> 7 & 63];
+    if (p.M == M && p.N == N && p.K == K && p.wt == wt) return p;
+    p = GemmPlan();
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    p.wt = wt;
+    if (tile_ok(K)) p.tile = tile_plan(M, N, K, wt);
+    if (gemm_skinny_ok(M, N, K, wt)) {
+        p.sk = sk_plan(M, N, K, wt);
+        const double e = p.sk.us, t = tile_ok(K) ? p.tile.us : 1e30;
+        p.skinny = wt == TLHIP_F16 ? 3.0 + 0.5 * e < t - 1.0 : (wt == TLHIP_Q8_0 ? e + 0.7 < t : 1.2 * e + 0.3 < t);
+    }
+    p.ws_bytes = p.skinny ? (p.sk.splits > 1 ? (size_t)p.sk.splits * M * N * sizeof(float) : 0) : p.tile.ws_bytes;
+    return p;
 }
 
 template <int WT, int MT, int NT, int KP>
@@ -908,287 +677,22 @@ static void launch_skinny(hipStream_t s, const GemmParams& p, const SkPlan& pl) 
     }
 }
 
-template <int WT, int BM, int BN, int NS>
-__global__ __launch_bounds__(512) void gemm_lds_kernel(GemmParams p, float* __restrict__ part, int mT, int nT, int splits) {
-    using L = Gl<WT, BM, BN, NS>;
-    constexpr int TM = BM / 64, TN = BN / 128;   // 32x32 tiles per wave
-    constexpr int WTN = BN / 4;                   // wave tile width
-    static_assert(TN >= 1 && BN % 128 == 0, "BN");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * L::STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 2, wn = wave & 3, hh = lane >> 5, l32 = lane & 31;
-    const int T = mT * nT;
-    const int q = gl_tile((int)blockIdx.x, T * splits);
-    const int z = q / T, qt = q % T;
-    const int m0 = (qt % mT) * BM, n0 = (qt / mT) * BN;
-    const int nkt = p.K / 64;
-    const int kt0 = (int)((int64_t)nkt * z / splits), kt1 = (int)((int64_t)nkt * (z + 1) / splits);
-    const int nk = kt1 - kt0;
-    const int nbr = p.K >> 5;
-
-    using DA = GlDma<L::A_BYTES>;
-    using DB = GlDma<L::B_BYTES>;
-    const uint8_t* a_src[DA::N];
-#pragma unroll
-    for (int u = 0; u < DA::N; u++) {
-        const int P = (u * 8 + wave) * 64 * DA::SZ + lane * DA::SZ;
-        const int r = P >> 7, c = ((P >> 4) & 7) ^ ((r >> 1) & 7);
-        const int m = min(m0 + r, p.M - 1);
-        a_src[u] = (const uint8_t*)(p.x + (size_t)m * p.K + (size_t)kt0 * 64 + 8 * c) + (P & 15);
-    }
-    const uint8_t* b_src[DB::N];
-#pragma unroll
-    for (int u = 0; u < DB::N; u++) {
-        constexpr int RB = GlRow<WT>::B;
-        const int P = (u * 8 + wave) * 64 * DB::SZ + lane * DB::SZ;
-        const int r = P / RB, cp = (P % RB) >> 4, byte = P & 15;
-        const int n = min(n0 + r, p.N - 1);
-        if (WT == TLHIP_F16) {
-            b_src[u] = p.wq + ((size_t)n * p.K + (size_t)kt0 * 64 + 8 * (cp ^ ((r >> 1) & 7))) * 2 + byte;
-        } else if (WT == TLHIP_Q8_0) {
-            b_src[u] = p.wq + (size_t)n * p.K + (size_t)kt0 * 64 + 16 * (cp ^ ((r >> 2) & 3)) + byte;
-        } else {
-            b_src[u] = p.wq + (size_t)n * (p.K / 2) + (size_t)kt0 * 32 + 16 * (cp ^ ((r >> 3) & 1)) + byte;
-        }
-    }
-    // scales: wave w, lanes < BN/8 -> row w*BN/8 + lane, both blocks of the step (4 bytes)
-    constexpr int SR = BN / 8;
-    const bool s_lane = lane < SR;
-    const uint8_t* s_src = nullptr;
-    if (L::S_BYTES) {
-        const int n = min(n0 + wave * SR + (s_lane ? lane : 0), p.N - 1);
-        s_src = (const uint8_t*)(p.wd + (size_t)n * nbr + 2 * (size_t)kt0);
-    }
-    constexpr int B_STEP = GlRow<WT>::B == 128 ? 128 : GlRow<WT>::B;
-
-    auto issue = [&](int step, int s) {   // step = kt - kt0
-        uint8_t* st = smem + s * L::STAGE;
-#pragma unroll
-        for (int u = 0; u < DA::N; u++) gl_dma<DA::SZ>(a_src[u] + (size_t)step * 128, st + (u * 8 + wave) * 64 * DA::SZ);
-#pragma unroll
-        for (int u = 0; u < DB::N; u++)
-            gl_dma<DB::SZ>(b_src[u] + (size_t)step * B_STEP, st + L::A_BYTES + (u * 8 + wave) * 64 * DB::SZ);
-        if (L::S_BYTES && s_lane) gl_dma<4>(s_src + (size_t)step * 4, st + L::A_BYTES + L::B_BYTES + wave * SR * 4);
-    };
-
-    f16v acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f16v{0};
-
-#pragma unroll
-    for (int s = 0; s < NS - 1; s++)
-        if (s < nk) issue(s, s);
-
-    // per-lane LDS offsets inside a stage (constant over the K loop)
-    int a_off[TM][4], b_off[TN][4];
-#pragma unroll
-    for (int ii = 0; ii < TM; ii++) {
-        const int m = wm * (BM / 2) + 32 * ii + l32;
-#pragma unroll
-        for (int t = 0; t < 4; t++) a_off[ii][t] = 128 * m + 16 * ((4 * hh + t) ^ ((m >> 1) & 7));
-    }
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const int n = wn * WTN + 32 * j + l32;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (WT == TLHIP_F16) b_off[j][t] = L::A_BYTES + 128 * n + 16 * ((4 * hh + t) ^ ((n >> 1) & 7));
-            else if (WT == TLHIP_Q8_0) b_off[j][t] = t < 2 ? L::A_BYTES + 64 * n + 16 * ((2 * hh + t) ^ ((n >> 2) & 3))
-                                                           : L::A_BYTES + L::B_BYTES + 4 * n + 2 * hh;
-            else b_off[j][t] = t == 0 ? L::A_BYTES + 32 * n + 16 * (hh ^ ((n >> 3) & 1))
-                                      : L::A_BYTES + L::B_BYTES + 4 * n + 2 * hh;
-        }
-    }
-
-    for (int i = 0; i < nk; i++) {
-        gl_wait_stage<L::VMC, NS - 2>(min(nk - 1 - i, NS - 2));
-        lds_barrier();   // stage i landed for every wave; stage i-1 fully read
-        if (i + NS - 1 < nk) issue(i + NS - 1, (i + NS - 1) % NS);
-
-        const uint8_t* st = smem + (i % NS) * L::STAGE;
-        // all LDS reads of the step first, then dequantise, then the MFMAs
-        h8 aop[TM][4];
-#pragma unroll
-        for (int ii = 0; ii < TM; ii++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) aop[ii][t] = *(const h8*)(st + a_off[ii][t]);
-        h8 bop[TN][4];
-        if (WT == TLHIP_F16) {
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int t = 0; t < 4; t++) bop[j][t] = *(const h8*)(st + b_off[j][t]);
-        } else if (WT == TLHIP_Q8_0) {
-            u4 raw[TN][2];
-            h16 dh[TN];
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                raw[j][0] = *(const u4*)(st + b_off[j][0]);
-                raw[j][1] = *(const u4*)(st + b_off[j][1]);
-                dh[j] = *(const h16*)(st + b_off[j][2]);
-            }
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const h2 dd = {dh[j], dh[j]};
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    uint32_t o0, o1, o2, o3;
-                    q8_pairs(raw[j][t >> 1][2 * (t & 1)], dd, o0, o1);
-                    q8_pairs(raw[j][t >> 1][2 * (t & 1) + 1], dd, o2, o3);
-                    bop[j][t] = __builtin_bit_cast(h8, u4{o0, o1, o2, o3});
-                }
-            }
-        } else {
-            u4 raw[TN];
-            h16 dh[TN];
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                raw[j] = *(const u4*)(st + b_off[j][0]);
-                dh[j] = *(const h16*)(st + b_off[j][1]);
-            }
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const h2 dd = {dh[j], dh[j]};
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    // t = 0/1: low nibbles of bytes 0-7 / 8-15; t = 2/3: high nibbles
-                    const uint32_t w0 = raw[j][2 * (t & 1)], w1 = raw[j][2 * (t & 1) + 1];
-                    const uint32_t n0w = t < 2 ? (w0 & 0x0F0F0F0Fu) : ((w0 >> 4) & 0x0F0F0F0Fu);
-                    const uint32_t n1w = t < 2 ? (w1 & 0x0F0F0F0Fu) : ((w1 >> 4) & 0x0F0F0F0Fu);
-                    uint32_t o0, o1, o2, o3;
-                    q4_pairs(n0w, dd, o0, o1);
-                    q4_pairs(n1w, dd, o2, o3);
-                    bop[j][t] = __builtin_bit_cast(h8, u4{o0, o1, o2, o3});
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int ii = 0; ii < TM; ii++)
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-                    acc[ii][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[ii][t], bop[j][t], acc[ii][j], 0, 0, 0);
-    }
-
-    // C layout: col = lane%32 (weight row n), row = 8*(r/4) + 4*(lane/32) + r%4 (activation row m)
-#pragma unroll
-    for (int ii = 0; ii < TM; ii++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn * WTN + 32 * j + l32;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * (BM / 2) + 32 * ii + 8 * (r >> 2) + 4 * hh + (r & 3);
-                const float v = acc[ii][j][r];
-                if (part) {
-                    if (m < p.M && n < p.N) part[((size_t)z * p.M + m) * p.N + n] = v;
-                } else {
-                    gemm_store_one(p, m, n, v);
-                }
-            }
-        }
-}
-
-// Sum of the split-K partials in slice order, then the epilogue.
-__global__ void gemm_reduce_kernel(GemmParams p, const float* __restrict__ part, int splits) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = (int64_t)p.M * p.N;
-    if (i >= total) return;
-    const int m = (int)(i / p.N), n = (int)(i % p.N);
-    float v = part[i];
-    for (int z = 1; z < splits; z++) v += part[(size_t)z * total + i];
-    if (p.epi == EPI_SWIGLU_PAIR) {
-        if ((n & 1) == 0 && n + 1 < p.N) {
-            float up = part[i + 1];
-            for (int z = 1; z < splits; z++) up += part[(size_t)z * total + i + 1];
-            p.y[(size_t)m * p.ldy + n / 2] = swiglu_h(f2h(v), f2h(up));
-        }
-    } else {
-        p.y[(size_t)m * p.ldy + n] = epilogue_h(p.epi, v, p.bias, p.resid, (size_t)m * p.N + n, n);
-    }
-}
-
-// gemm_reduce_kernel for 4 consecutive columns per thread (16-byte partial
-// loads, one 8-byte store; the SwiGLU pair epilogue: two outputs, one
-// 4-byte store): the same sums in slice order and the same epilogue per
-// element.  N and the output row stride multiples of 4 (SwiGLU: of 2 for
-// the output), the partials 16-byte and the other pointers 8-byte aligned.
-__global__ void gemm_reduce4_kernel(GemmParams p, const float* __restrict__ part, int splits) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    const int64_t total = (int64_t)p.M * p.N;
-    if (i >= total) return;
-    const int m = (int)(i / p.N), n = (int)(i % p.N);
-    float4 v = *(const float4*)(part + i);
-    for (int z = 1; z < splits; z++) {
-        const float4 t = *(const float4*)(part + (size_t)z * total + i);
-        v.x += t.x;
-        v.y += t.y;
-        v.z += t.z;
-        v.w += t.w;
-    }
-    if (p.epi == EPI_SWIGLU_PAIR) {
-        const uint32_t o0 = swiglu_h(f2h(v.x), f2h(v.y)), o1 = swiglu_h(f2h(v.z), f2h(v.w));
-        *(uint32_t*)(p.y + (size_t)m * p.ldy + n / 2) = o0 | (o1 << 16);
-        return;
-    }
-    const size_t ri = (size_t)m * p.N + n;
-    const uint32_t o0 = epilogue_h(p.epi, v.x, p.bias, p.resid, ri, n);
-    const uint32_t o1 = epilogue_h(p.epi, v.y, p.bias, p.resid, ri + 1, n + 1);
-    const uint32_t o2 = epilogue_h(p.epi, v.z, p.bias, p.resid, ri + 2, n + 2);
-    const uint32_t o3 = epilogue_h(p.epi, v.w, p.bias, p.resid, ri + 3, n + 3);
-    *(uint2*)(p.y + (size_t)m * p.ldy + n) = uint2{o0 | (o1 << 16), o2 | (o3 << 16)};
-}
-
-constexpr int GL_BM = 128, GL_BN = 128;
-
-template <int WT>
-static void launch_gemm2(hipStream_t s, const GemmParams& p, int splits, float* part) {
-    if (p.M > 64) {
-        // four stages (one workgroup per CU) while the grid fits the 256 CUs;
-        // beyond that three stages, so that two workgroups share a CU
-        const int mT = (p.M + GL_BM - 1) / GL_BM, nT = (p.N + GL_BN - 1) / GL_BN;
-        const unsigned grid = (unsigned)(mT * nT * splits);
-        if (grid > 256)
-            hipLaunchKernelGGL((gemm_lds_kernel<WT, GL_BM, GL_BN, 3>), dim3(grid), dim3(512), 0, s, p, part, mT, nT, splits);
-        else
-            hipLaunchKernelGGL((gemm_lds_kernel<WT, GL_BM, GL_BN, 4>), dim3(grid), dim3(512), 0, s, p, part, mT, nT, splits);
-    } else {
-        dim3 grid((unsigned)((p.N + 63) / 64), (unsigned)((p.M + 63) / 64), (unsigned)splits);
-        hipLaunchKernelGGL((gemm2_kernel<WT, 64, 64, 2, 2>), grid, dim3(256), 0, s, p, part);
-    }
-}
-
-// split-K slices.  M <= 64 (register-staged 64 x 64 tiles): enough
-// workgroups to cover the 256 CUs about once, at least 4 K steps per slice.
-// M > 64 (multi-stage 128 x 128 tiles, one workgroup per CU): up to 4
-// slices while the grid stays within 320 workgroups, at least 8 K steps
-// per slice.
-// The bound GEMM_SPLIT_PARTIALS_MAX states for each branch below (the fixed
-// workspace of the no-allocation entry point is sized by it).
-static_assert((size_t)GEMM_SPLIT_TILE_CAP * GL_BM * GL_BN * sizeof(float) <= GEMM_SPLIT_PARTIALS_MAX, "M > 64 split");
+// The bounds GEMM_SPLIT_PARTIALS_MAX states (the fixed workspace of the
+// no-allocation entry point is sized by it); tile_plan keeps to it itself.
 static_assert((size_t)SK_MAX_SPLITS * 64 * (SK_MAX_TILES_SPLIT * 16 * 4) * sizeof(float) <= GEMM_SPLIT_PARTIALS_MAX,
               "skinny split (64 rows, N <= SK_MAX_TILES_SPLIT tiles of 16 x 4 weight rows)");
-static_assert((size_t)512 * 64 * 64 * sizeof(float) <= GEMM_SPLIT_PARTIALS_MAX, "M <= 64 split");
-int gemm_splits(int M, int N, int K, int wt) {
-    if (wt < 0) {   // any weight type: the largest count any of them takes
-        int sp = 1;
-        for (int t : {(int)TLHIP_F16, (int)TLHIP_Q8_0, (int)TLHIP_Q4_0, (int)TLHIP_Q6_K}) sp = std::max(sp, gemm_splits(M, N, K, t));
-        return sp;
+
+size_t gemm_ws_bytes(int M, int N, int K, int wt) {
+    if (wt < 0) {
+        size_t b = 0;
+        for (int t : {(int)TLHIP_F16, (int)TLHIP_Q8_0, (int)TLHIP_Q4_0}) b = std::max(b, gemm_ws_bytes(M, N, K, t));
+        return b;
     }
-    if (gemm_skinny_ok(M, N, K, wt)) return sk_plan(M, N, K, wt).splits;
-    if (K % G2_BK) return 1;
-    int sp = 1;
-    if (M > 64) {
-        const int tiles = ((N + GL_BN - 1) / GL_BN) * ((M + GL_BM - 1) / GL_BM);
-        while (sp < 4 && tiles * sp * 2 <= GEMM_SPLIT_TILE_CAP && (K / G2_BK) / (sp * 2) >= 8) sp *= 2;
-        return sp;
-    }
-    const int tiles = ((N + 63) / 64) * ((M + 63) / 64);
-    while (sp < 8 && tiles * sp * 2 <= 512 && (K / G2_BK) / (sp * 2) >= 4) sp *= 2;
-    return sp;
+    return gemm_plan(M, N, K, wt).ws_bytes;
+}
+
+bool gemm_rope_ok(int M, int N, int K, int wt) {
+    return (wt == TLHIP_F16 || wt == TLHIP_Q8_0 || wt == TLHIP_Q4_0) && tile_ok(K);
 }
 
 // Naive fp32-accumulate GEMM for f16 weights whose K is not a multiple of 32
@@ -1220,10 +724,10 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
     if (a.pro != PRO_NONE)
         return fail(TLHIP_ERR_INVALID_OPERATION, "gemm: the fused normalisation prologue is GEMV-only");
     if (epi == EPI_QKV_ROPE) {
-        if (!gemm_skinny_ok(p.M, p.N, p.K, wt) || a.d_pos || !a.rope_tab || !a.q_out || !a.kc || !a.vc ||
+        if (!gemm_rope_ok(p.M, p.N, p.K, wt) || a.d_pos || !a.rope_tab || !a.q_out || !a.kc || !a.vc ||
             a.head_dim <= 0 || a.head_dim % 2 || a.rot % 2 || a.rot > a.head_dim || a.nq % a.head_dim ||
             a.nk % a.head_dim || a.nq + 2 * a.nk != p.N)
-            return fail(TLHIP_ERR_INVALID_OPERATION, "gemm: the RoPE epilogue needs the skinny GEMM and a q/k/v layout");
+            return fail(TLHIP_ERR_INVALID_OPERATION, "gemm: the RoPE epilogue needs K %% 32 == 0 and a q/k/v layout");
         p.nq = a.nq;
         p.nk = a.nk;
         p.head_dim = a.head_dim;
@@ -1245,10 +749,11 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
         hipLaunchKernelGGL(gemm_naive_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p);
         return TLHIP_OK;
     }
-    if (gemm_skinny_ok(p.M, p.N, p.K, wt)) {
+    const GemmPlan& plan = gemm_plan(p.M, p.N, p.K, wt);
+    if (plan.skinny) {
         // K split over workgroups only with a workspace for the partials and
         // the per-tile counters
-        const SkPlan pl = sk_plan(p.M, p.N, p.K, wt);
+        const SkPlan& pl = plan.sk;
         p.mtiles = pl.mtiles;
         if (pl.splits > 1 && a.ws && a.tile_flags && (size_t)pl.splits * p.M * p.N * sizeof(float) <= a.ws_bytes) {
             p.splits = pl.splits;
@@ -1260,26 +765,7 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
         else launch_skinny<TLHIP_F16>(s, p, pl);
         return TLHIP_OK;
     }
-    if (p.K % G2_BK == 0) {
-        int splits = a.ws ? gemm_splits(p.M, p.N, p.K, wt) : 1;
-        if ((size_t)splits * p.M * p.N * sizeof(float) > a.ws_bytes) splits = 1;
-        float* part = splits > 1 ? a.ws : nullptr;
-        if (wt == TLHIP_Q4_0) launch_gemm2<TLHIP_Q4_0>(s, p, splits, part);
-        else if (wt == TLHIP_Q8_0) launch_gemm2<TLHIP_Q8_0>(s, p, splits, part);
-        else launch_gemm2<TLHIP_F16>(s, p, splits, part);
-        if (splits > 1) {
-            const int64_t total = (int64_t)p.M * p.N;
-            const bool vec = p.N % 4 == 0 && p.ldy % (p.epi == EPI_SWIGLU_PAIR ? 2 : 4) == 0 &&
-                             ((uintptr_t)p.y | (uintptr_t)p.bias | (uintptr_t)p.resid) % 8 == 0 && (uintptr_t)part % 16 == 0;
-            if (vec)
-                hipLaunchKernelGGL(gemm_reduce4_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, s, p,
-                                   (const float*)part, splits);
-            else
-                hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p,
-                                   (const float*)part, splits);
-        }
-        return TLHIP_OK;
-    }
+    if (tile_ok(p.K)) return launch_gemm_tile(s, wt, a, epi, p.ldy, plan.tile);
     dim3 grid((unsigned)((p.N + GBN - 1) / GBN), (unsigned)((p.M + GBM - 1) / GBM));
     if (wt == TLHIP_Q4_0) hipLaunchKernelGGL(gemm_kernel<TLHIP_Q4_0>, grid, dim3(256), 0, s, p);
     else if (wt == TLHIP_Q8_0) hipLaunchKernelGGL(gemm_kernel<TLHIP_Q8_0>, grid, dim3(256), 0, s, p);

@@ -1,0 +1,148 @@
+// kernels_gemm_tile.hip -- launches of the tiled MFMA dequant-GEMM
+// (gemm_tile.hpp): tile shape and K split by a cost model, and the sum of the
+// K slices.
+#include <algorithm>
+
+#include "gemm_tile.hpp"
+
+namespace tlhip {
+
+// The K slices' partials summed in slice order, then the epilogue: 8
+// consecutive outputs per thread.  Bound by the partials' bytes (M = 512, N =
+// 2560, 3 slices: 15.7 MB, 5.5 us).
+__global__ __launch_bounds__(256) void tile_reduce_kernel(TileParams p) {
+    const int per_row = (p.N + 7) / 8;
+    const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (it >= (int64_t)p.M * per_row) return;
+    const int m = (int)(it / per_row), n = (int)(it % per_row) * 8;
+    const size_t row = (p.N + 7) & ~7, total = (size_t)p.M * row;
+    const float* s = p.part + m * row + n;
+    f4 a = *(const f4*)s, b = *(const f4*)(s + 4);
+    for (int z = 1; z < p.splits; z++) {
+        a += *(const f4*)(s + z * total);
+        b += *(const f4*)(s + z * total + 4);
+    }
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+    }
+    tile_store8(p, m, n, v);
+}
+
+namespace {
+
+// Tile shapes.  A wave of 128 x 64 dequantises each weight once; the smaller
+// ones fill more CUs.  (Measured and not built: 128 x 128 in 64 x 64 waves,
+// within 4 % of the first for f16 weights and behind for packed ones; 32 x 64
+// for M <= 32, never more than 3 % ahead of 64 x 32.)
+struct TileShape {
+    int bm, bn, bk;
+    float fix;    // us per round of workgroups: first loads, epilogue
+    float kbus;   // KB of a stage that a step streams per us, few CUs busy
+    float load;   // slowdown per step with all 256 CUs busy
+};
+constexpr TileShape SHAPES[5] = {
+    {128, 128, 128, 5.2f, 85.0f, 0.42f}, {128, 64, 128, 1.7f, 84.0f, 0.30f}, {64, 128, 128, 3.4f, 84.0f, 0.30f},
+    {64, 64, 256, 2.25f, 84.0f, 0.30f},  {64, 32, 256, 0.95f, 84.0f, 0.30f},
+};
+
+double stage_kb(const TileShape& t, int wt) {
+    const int blocks = t.bk / 32, wb = wt == TLHIP_F16 ? 64 : (wt == TLHIP_Q8_0 ? 32 : 16);
+    return (t.bm * t.bk * 2.0 + (double)t.bn * wb * blocks + (wt == TLHIP_F16 ? 0.0 : t.bn * (blocks / 2 + 1) * 4.0)) / 1024.0;
+}
+
+}  // namespace
+
+// Tile shape and K slices for (M, N, K, weight type).  The model is fitted to
+// measurements of every shape and split on 114 problems (M 5 - 2048, N 64 -
+// 32000, K 256 - 10240, the three weight types): a launch costs 2.9 us, plus
+// per round of 256 workgroups (one per CU: the ring fills the LDS) its fixed
+// part and its steps, each the time its bytes stream in at; a split adds 3.1
+// us and its partials' traffic.  The pick is 0.7 % slower than the best
+// measured one on average, 17 % at worst.
+TilePlan tile_plan(int M, int N, int K, int wt) {
+    TilePlan best;
+    double best_us = 1e30;
+    for (int c = 0; c < 5; c++) {
+        const TileShape& t = SHAPES[c];
+        const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const int steps = (K + t.bk - 1) / t.bk;
+        for (int sp : {1, 2, 3, 4, 6, 8}) {
+            const size_t bytes = (size_t)sp * M * ((N + 7) & ~7) * sizeof(float);
+            if (sp > 1 && (tiles * sp > 320 || steps / sp < 2 || bytes > GEMM_SPLIT_PARTIALS_MAX)) break;
+            const int64_t wgs = tiles * sp;
+            const double busy = (double)std::min<int64_t>(wgs, 256);
+            const double step_us = stage_kb(t, wt) / t.kbus * (1.0 + t.load * std::max(0.0, busy - 64.0) / 192.0);
+            double us = 2.9 + (double)((wgs + 255) / 256) * (t.fix + (steps + sp - 1) / sp * step_us);
+            if (sp > 1) us += 3.1 + (sp * 4.0 + 2.0) * M * N / 4.3e6;
+            if (us < best_us) {
+                best_us = us;
+                best.shape = c;
+                best.splits = sp;
+                best.ws_bytes = sp > 1 ? bytes : 0;
+            }
+        }
+    }
+    best.us = best_us;
+    return best;
+}
+
+template <int WT, int TM, int TN, int WM, int WN>
+static void launch_tile(hipStream_t s, TileParams& p) {
+    using L = Tile<WT, TM, TN, WM, WN, 1>;
+    p.mT = (p.M + L::BM - 1) / L::BM;
+    p.nT = (p.N + L::BN - 1) / L::BN;
+    hipLaunchKernelGGL((gemm_tile_kernel<WT, TM, TN, WM, WN, 1>), dim3((unsigned)(p.mT * p.nT * p.splits)), dim3(512), 0, s, p);
+}
+template <int WT>
+static void launch_shape(hipStream_t s, TileParams& p, int shape) {
+    switch (shape) {
+        case 0: launch_tile<WT, 4, 2, 1, 2>(s, p); break;
+        case 1: launch_tile<WT, 2, 2, 2, 1>(s, p); break;
+        case 2: launch_tile<WT, 2, 2, 1, 2>(s, p); break;
+        case 3: launch_tile<WT, 2, 2, 1, 1>(s, p); break;
+        default: launch_tile<WT, 2, 1, 1, 1>(s, p); break;
+    }
+}
+
+tlhip_status launch_gemm_tile(hipStream_t s, int wt, const GemvArgs& a, int epi, int ldy, const TilePlan& pl) {
+    TileParams p = {};
+    p.x = a.x;
+    p.wq = (const uint8_t*)a.wq;
+    p.wd = a.wd;
+    p.bias = a.bias;
+    p.resid = a.resid;
+    p.y = a.y;
+    p.M = a.M;
+    p.N = a.N;
+    p.K = a.K;
+    p.ldy = ldy;
+    p.epi = epi;
+    p.splits = pl.splits > 1 && a.ws && pl.ws_bytes <= a.ws_bytes && (uintptr_t)a.ws % 16 == 0 ? pl.splits : 1;
+    p.part = p.splits > 1 ? a.ws : nullptr;
+    if (epi == EPI_QKV_ROPE) {
+        p.nq = a.nq;
+        p.nk = a.nk;
+        p.head_dim = a.head_dim;
+        p.rot = a.rot;
+        p.layout = a.layout;
+        p.pos0 = a.pos0;
+        p.rope_tab = a.rope_tab;
+        p.q_out = a.q_out;
+        p.kc = a.kc;
+        p.vc = a.vc;
+        p.vec = a.head_dim % 8 == 0 && a.rot % 8 == 0 && ((uintptr_t)a.q_out | (uintptr_t)a.kc | (uintptr_t)a.vc) % 16 == 0;
+    }
+    if (wt == TLHIP_Q4_0) launch_shape<TLHIP_Q4_0>(s, p, pl.shape);
+    else if (wt == TLHIP_Q8_0) launch_shape<TLHIP_Q8_0>(s, p, pl.shape);
+    else launch_shape<TLHIP_F16>(s, p, pl.shape);
+    if (p.splits > 1) {
+        const int64_t items = (int64_t)p.M * ((p.N + 7) / 8);
+        hipLaunchKernelGGL(tile_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, p);
+    }
+    return TLHIP_OK;
+}
+
+}  // namespace tlhip

@@ -412,7 +412,7 @@ tlhip_status enqueue_forward(tlhip_model m, int S, int pos0, const int32_t* ids_
         } else {
             if (m->arch == 0) TLHIP_TRY(launch_rms_norm(s, P(m->x), P(L.norm_w), P(m->xn), S, H, m->eps));
             else TLHIP_TRY(launch_layer_norm(s, P(m->x), P(L.norm_w), P(L.norm_b), P(m->xn), S, H, m->eps));
-            if (!decode && gemm_skinny_ok(S, qkv_w, H, L.qkv.w->dtype)) {
+            if (!decode && gemm_rope_ok(S, qkv_w, H, L.qkv.w->dtype)) {
                 // qkv (+ bias) + RoPE + cache write in the GEMM's epilogue
                 GemvArgs a;
                 a.x = P(m->xn);
@@ -960,10 +960,7 @@ tlhip_status tlhip_model_load(tlhip_ctx ctx, const char* path, int arch, int max
             const int64_t shapes[4][2] = {{H + 2 * kvd, H}, {H, H}, {arch == 0 ? 2 * I : I, H}, {H, I}};
             size_t need = 0;
             for (int rows = 5; rows <= (int)R; rows++)
-                for (auto& sh : shapes) {
-                    const int sp = gemm_splits(rows, (int)sh[0], (int)sh[1], -1);
-                    if (sp > 1) need = std::max(need, (size_t)sp * rows * sh[0] * sizeof(float));
-                }
+                for (auto& sh : shapes) need = std::max(need, gemm_ws_bytes(rows, (int)sh[0], (int)sh[1], -1));
             if (need) {
                 e = hipMalloc(&m->ws, need);
                 m->ws_bytes = need;

@@ -10,7 +10,7 @@
 // per device; host code only ever passes that address, never the array's
 // name, to kernels.
 //
-// The split is the one tlhip_linear picks (gemm_splits), so both entry points
+// The split is the one tlhip_linear picks (gemm_ws_bytes), so both entry points
 // run the same kernels and produce the same bits.  Every partial a reduction
 // reads is written by the GEMM of the same call (each slice covers every
 // output element of its tiles), so the contents a previous call left behind
@@ -25,10 +25,7 @@
 
 namespace {
 
-// Largest split-K partial set gemm_splits can ask for (GEMM_SPLIT_PARTIALS_MAX,
-// 20 MiB: M > 64 keeps at most 320 tiles of 128 x 128 over all slices, e.g.
-// Q4_0 [512 x 10240] @ [2560 x 10240]^T in 4 slices; the skinny GEMM's
-// splits stay within 16 MiB).
+// The largest split-K partial set any plan asks for.
 constexpr size_t kScratchBytes = tlhip::GEMM_SPLIT_PARTIALS_MAX;
 constexpr int kMaxDevices = 64;
 

@@ -189,9 +189,8 @@ tlhip_status linear_impl(tlhip_ctx ctx, tlhip_tensor x, tlhip_tensor w, tlhip_te
     // MFMA GEMM; a split-K workspace when the output has too few tiles to
     // fill the device: the context's, grown (stream-ordered) when a call
     // needs more, so steady-state calls allocate nothing
-    const int sp = gemm_splits((int)M, (int)N, (int)K, (int)wt);
-    const size_t need = (size_t)sp * M * N * sizeof(float);
-    if (sp > 1 && no_alloc) {
+    const size_t need = gemm_ws_bytes((int)M, (int)N, (int)K, (int)wt);
+    if (need && no_alloc) {
         // the caller's fixed workspace: the same split as the pool path, so
         // the same kernels and the same bits
         if (need > fixed_ws_bytes)
@@ -200,7 +199,7 @@ tlhip_status linear_impl(tlhip_ctx ctx, tlhip_tensor x, tlhip_tensor w, tlhip_te
                         "workspace of %zu bytes", need, (long long)M, (long long)N, fixed_ws_bytes);
         a.ws = fixed_ws;
         a.ws_bytes = need;
-    } else if (sp > 1) {
+    } else if (need) {
         if (float* ws = ctx_workspace(ctx, need)) {   // (none: the GEMM runs unsplit)
             a.ws = ws;
             a.ws_bytes = need;

@@ -175,7 +175,8 @@ tlhip_status alloc_tensor(tlhip_ctx ctx, tlhip_dtype dtype, int ndim, const int6
             return fail(TLHIP_ERR_INVALID_DIMENSION, "quantized tensors must be 2-D [N, K] with K %% %d == 0",
                         (int)quant_group(dtype));
         qs_bytes = quant_data_bytes(dtype, shape[0], shape[1]);
-        bytes = qs_bytes + (size_t)quant_scale_count(dtype, shape[0], shape[1]) * 2;
+        // (whole 4-byte words: the GEMM loads scales in pairs)
+        bytes = (qs_bytes + (size_t)quant_scale_count(dtype, shape[0], shape[1]) * 2 + 3) & ~(size_t)3;
     }
     auto* t = new tlhip_tensor_s();
     t->ctx = ctx;
