@@ -16,6 +16,15 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 constexpr int WAVE = 64;
 
+// 8 (4) f16 values at any 2-byte aligned address, one access where the
+// hardware takes it unaligned (rows of an odd length are).
+struct __attribute__((packed, aligned(2))) h8_any {
+    uint32_t w[4];
+};
+struct __attribute__((packed, aligned(2))) h4_any {
+    uint32_t w[2];
+};
+
 __device__ __forceinline__ float h2f(uint16_t b) { return (float)__builtin_bit_cast(h16, b); }
 // v_cvt_f16_f32: round-to-nearest-even, f16 denormals preserved.
 __device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, (h16)f); }

@@ -202,15 +202,6 @@ __device__ __forceinline__ void tile_rope8(const TileParams& p, int m, int n, ui
     }
 }
 
-// 8 (4) f16 values at any 2-byte aligned address, one access where the
-// hardware takes it unaligned (rows of an odd length are).
-struct __attribute__((packed, aligned(2))) h8_any {
-    uint32_t w[4];
-};
-struct __attribute__((packed, aligned(2))) h4_any {
-    uint32_t w[2];
-};
-
 // The epilogue (GemvEpi) of 8 consecutive outputs n .. n + 7 of row m (the
 // last item of a row may hold fewer).
 __device__ __forceinline__ void tile_store8(const TileParams& p, int m, int n, const float (&v)[8]) {

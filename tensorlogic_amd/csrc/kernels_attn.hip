@@ -1926,8 +1926,9 @@ __global__ __launch_bounds__(256) void context8_kernel(const uint16_t* __restric
     if (tid < D) out[(size_t)row * D + tid] = f2h(((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid]);
 }
 
-// The 8-lane kernels for D = 64 / 80 / 128 on 4-byte aligned tensors, the
-// one-output-per-thread kernels otherwise.
+// The matrix cores for many rows (kernels_einsum.hip), the 8-lane kernels for
+// D = 64 / 80 / 128 on 4-byte aligned tensors, the one-output-per-thread
+// kernels otherwise.
 static bool einsum8_ok(const void* a, const void* b, int D) {
     return (D == 64 || D == 80 || D == 128) && ((uintptr_t)a & 3) == 0 && ((uintptr_t)b & 3) == 0;
 }
@@ -1936,6 +1937,7 @@ tlhip_status launch_scores(hipStream_t s, const uint16_t* q, const uint16_t* k, 
                            int J, int H, int Hkv, int D) {
     int64_t n = (int64_t)I * H * J;
     if (n <= 0) return TLHIP_OK;
+    if (launch_scores_mfma(s, q, k, sc, I, J, H, Hkv, D)) return TLHIP_OK;
     if (einsum8_ok(q, k, D)) {
         const dim3 grid((unsigned)((n + 31) / 32));
         if (D == 64) hipLaunchKernelGGL(scores8_kernel<64>, grid, dim3(256), 0, s, q, k, sc, I, J, H, Hkv);
@@ -1952,6 +1954,7 @@ tlhip_status launch_context(hipStream_t s, const uint16_t* p, const uint16_t* v,
                             int J, int H, int Hkv, int D) {
     int64_t n = (int64_t)I * H * D;
     if (n <= 0) return TLHIP_OK;
+    if (launch_context_mfma(s, p, v, out, I, J, H, Hkv, D)) return TLHIP_OK;
     if (J > 0 && einsum8_ok(p, v, D) && (int64_t)I * H <= 0x7fffffff) {
         const dim3 grid((unsigned)(I * H));
         if (D == 64) hipLaunchKernelGGL(context8_kernel<64>, grid, dim3(256), 0, s, p, v, out, J, H, Hkv);
