@@ -511,8 +511,83 @@ __global__ __launch_bounds__(256) void softmax_kernel(const uint16_t* __restrict
     }
 }
 
+// The same for rows of up to 1024 elements, one wave per row with the row in
+// registers: x is read once and y written once, with no workgroup barrier.
+// Lane l holds the C elements from C l on (C consecutive, and 512 further on
+// a second 8 for rows past 512): the smallest C that covers the row, so that
+// short rows spread over the lanes and long ones move 16 bytes per lane.
+// 12,800 rows of 400: 21.5 -> 12.3 us; 32 rows of 24: 3.4 -> 2.8.
+template <int C, int CHUNKS>
+__global__ __launch_bounds__(256) void softmax_wave_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
+                                                           int64_t rows, int n) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int lane = threadIdx.x & 63;
+    const uint16_t* xr = x + row * n;
+    uint16_t* yr = y + row * n;
+    float v[CHUNKS][C];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < CHUNKS; u++) {
+        const int i0 = C * (lane + 64 * u);
+        uint16_t h[C];
+        if (C == 8 && i0 + 8 <= n) {
+            const h8_any w = *(const h8_any*)(xr + i0);
+#pragma unroll
+            for (int e = 0; e < C; e++) h[e] = (uint16_t)(w.w[e / 2] >> (16 * (e & 1)));
+        } else {
+#pragma unroll
+            for (int e = 0; e < C; e++) h[e] = i0 + e < n ? xr[i0 + e] : (uint16_t)0xFC00u;   // -inf
+        }
+#pragma unroll
+        for (int e = 0; e < C; e++) {
+            v[u][e] = h2f(h[e]);
+            if (isfinite(v[u][e])) mx = fmaxf(mx, v[u][e]);
+        }
+    }
+    mx = wave_max(mx);
+    if (!isfinite(mx)) mx = 0.0f;
+    float sum = 0.0f;
+#pragma unroll
+    for (int u = 0; u < CHUNKS; u++)
+#pragma unroll
+        for (int e = 0; e < C; e++) {
+            const float t = isfinite(v[u][e]) ? expf(v[u][e] - mx) : 0.0f;
+            sum += t;
+            v[u][e] = h2f(f2h(t));
+        }
+    sum = wave_sum<64>(sum);
+    const bool ok = sum > 0.0f && isfinite(sum);
+#pragma unroll
+    for (int u = 0; u < CHUNKS; u++) {
+        const int i0 = C * (lane + 64 * u);
+        uint16_t o[C];
+#pragma unroll
+        for (int e = 0; e < C; e++) o[e] = f2h(ok ? v[u][e] / sum : 1.0f / (float)n);
+        if (C == 8 && i0 + 8 <= n) {
+            h8_any q;
+#pragma unroll
+            for (int e = 0; e + 1 < C; e += 2) q.w[e / 2] = (uint32_t)o[e] | ((uint32_t)o[e + 1] << 16);
+            *(h8_any*)(yr + i0) = q;
+        } else {
+#pragma unroll
+            for (int e = 0; e < C; e++)
+                if (i0 + e < n) yr[i0 + e] = o[e];
+        }
+    }
+}
+
 tlhip_status launch_softmax(hipStream_t s, const uint16_t* x, uint16_t* y, int64_t rows, int n) {
     if (rows <= 0 || n <= 0) return TLHIP_OK;
+    if (n <= 1024) {
+        const dim3 grid((unsigned)((rows + 3) / 4));
+        if (n <= 64) hipLaunchKernelGGL((softmax_wave_kernel<1, 1>), grid, dim3(256), 0, s, x, y, rows, n);
+        else if (n <= 128) hipLaunchKernelGGL((softmax_wave_kernel<2, 1>), grid, dim3(256), 0, s, x, y, rows, n);
+        else if (n <= 256) hipLaunchKernelGGL((softmax_wave_kernel<4, 1>), grid, dim3(256), 0, s, x, y, rows, n);
+        else if (n <= 512) hipLaunchKernelGGL((softmax_wave_kernel<8, 1>), grid, dim3(256), 0, s, x, y, rows, n);
+        else hipLaunchKernelGGL((softmax_wave_kernel<8, 2>), grid, dim3(256), 0, s, x, y, rows, n);
+        return TLHIP_OK;
+    }
     hipLaunchKernelGGL(softmax_kernel, dim3((unsigned)rows), dim3(256), 0, s, x, y, n);
     return TLHIP_OK;
 }
@@ -540,9 +615,49 @@ __global__ void elementwise_kernel(int op, const uint16_t* __restrict__ a,
     y[i] = r;
 }
 
+// Eight consecutive elements per thread, 16-byte accesses (n, and a row
+// broadcast's period, multiples of 8; 16-byte aligned tensors).  Bound by the
+// bytes: 5.1 M elements by a scalar, 9.4 -> 6.5 us.
+__global__ __launch_bounds__(256) void elementwise8_kernel(int op, const uint16_t* __restrict__ a,
+                                                           const uint16_t* __restrict__ b, uint16_t* __restrict__ y,
+                                                           int64_t n8, int64_t bp, float sc) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const u4 av = *(const u4*)(a + 8 * i);
+    u4 bv = {0u, 0u, 0u, 0u}, o;
+    if (op == EW_ADD || op == EW_MUL || op == EW_SILU_MUL) bv = *(const u4*)(b + (bp ? 8 * i % bp : 8 * i));
+    uint16_t r[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const uint16_t x = (uint16_t)(av[e / 2] >> (16 * (e & 1))), z = (uint16_t)(bv[e / 2] >> (16 * (e & 1)));
+        switch (op) {
+            case EW_SIGMOID: r[e] = sigmoid_h(x); break;
+            case EW_SILU: r[e] = f2h(h2f(x) * h2f(sigmoid_h(x))); break;
+            case EW_GELU: r[e] = gelu_h(x); break;
+            case EW_ADD: r[e] = f2h(h2f(x) + h2f(z)); break;
+            case EW_MUL: r[e] = f2h(h2f(x) * h2f(z)); break;
+            case EW_MUL_SCALAR: r[e] = f2h(h2f(x) * sc); break;
+            case EW_SILU_MUL: r[e] = swiglu_h(x, z); break;
+            default: r[e] = x;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = (uint32_t)r[2 * e] | ((uint32_t)r[2 * e + 1] << 16);
+    *(u4*)(y + 8 * i) = o;
+}
+
+// From 2^16 elements on, where the wide form still has a workgroup for half
+// the CUs; fewer are latency-bound either way.
+constexpr int64_t kWideElems = 1 << 16;
+
 tlhip_status launch_elementwise(hipStream_t s, int op, const uint16_t* a, const uint16_t* b,
                                 uint16_t* y, int64_t n, int64_t b_period, float scalar) {
     if (n <= 0) return TLHIP_OK;
+    if (n >= kWideElems && n % 8 == 0 && b_period % 8 == 0 && ((uintptr_t)a | (uintptr_t)b | (uintptr_t)y) % 16 == 0) {
+        hipLaunchKernelGGL(elementwise8_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, op, a, b, y, n / 8,
+                           b_period, scalar);
+        return TLHIP_OK;
+    }
     hipLaunchKernelGGL(elementwise_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, op, a,
                        b, y, n, b_period, scalar);
     return TLHIP_OK;
@@ -568,6 +683,27 @@ __global__ void mask_kernel(const uint16_t* __restrict__ sc, const uint16_t* __r
     y[i] = ((m & 0x7fffu) == 0) ? f2h(-10000.0f) : sc[i];
 }
 
+// Eight consecutive scores per thread, 5.1 M of them 12.2 -> 6.9 us (n, and the mask's period or row,
+// multiples of 8).
+__global__ __launch_bounds__(256) void mask8_kernel(const uint16_t* __restrict__ sc, const uint16_t* __restrict__ mask,
+                                                    uint16_t* __restrict__ y, int64_t n8, int64_t period, int64_t inner,
+                                                    int64_t heads) {
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g >= n8) return;
+    const int64_t i = 8 * g;
+    const int64_t mi = heads > 1 ? i / inner / heads * inner + i % inner : (period > i ? i : i % period);
+    const u4 m = *(const u4*)(mask + mi), v = *(const u4*)(sc + i);
+    const uint32_t off = f2h(-10000.0f);
+    u4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t lo = (m[e] & 0x7fffu) == 0 ? off : v[e] & 0xffffu;
+        const uint32_t hi = (m[e] & 0x7fff0000u) == 0 ? off << 16 : v[e] & 0xffff0000u;
+        o[e] = lo | hi;
+    }
+    *(u4*)(y + i) = o;
+}
+
 tlhip_status launch_mask(hipStream_t s, const uint16_t* sc, const uint16_t* mask, uint16_t* y,
                          int64_t n, int64_t mask_period) {
     // mask_period > 0: elementwise repeat; mask_period < 0 encodes (-J, H)
@@ -579,6 +715,12 @@ tlhip_status launch_mask(hipStream_t s, const uint16_t* sc, const uint16_t* mask
         inner = enc >> 16;
         heads = enc & 0xffff;
         period = 0;
+    }
+    if (n >= kWideElems && n % 8 == 0 && (heads > 1 ? inner : period) % 8 == 0 &&
+        ((uintptr_t)sc | (uintptr_t)mask | (uintptr_t)y) % 16 == 0) {
+        hipLaunchKernelGGL(mask8_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, sc, mask, y, n / 8,
+                           period, inner, heads);
+        return TLHIP_OK;
     }
     hipLaunchKernelGGL(mask_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, sc, mask, y, n,
                        period, inner, heads);
@@ -741,10 +883,70 @@ __global__ void broadcast_kernel(const T* __restrict__ x, T* __restrict__ y, int
     y[g] = x[src];
 }
 
-tlhip_status launch_broadcast(hipStream_t s, const void* x, void* y, int elem, const BcastDims& b) {
+// Eight f16 (four 32-bit) elements per thread, 32-bit index arithmetic
+// ([400, 1, 400] to 32 heads: 17.2 -> 5.4 us; K rows to GQA heads 5.9 -> 3.2): the
+// innermost dim a multiple of the vector and either contiguous or repeated.
+template <typename T>
+__global__ __launch_bounds__(256) void broadcast16_kernel(const T* __restrict__ x, T* __restrict__ y, uint32_t total,
+                                                          BcastDims b) {
+    constexpr int V = 16 / sizeof(T);
+    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
+    if (g >= total) return;
+    const int l = b.nd - 1;
+    uint32_t rem = g;
+    size_t src = 0;
+    {
+        const uint32_t per = (uint32_t)b.shape[l] / V;
+        src = (size_t)(rem % per) * V * b.xstride[l];
+        rem /= per;
+    }
+    for (int i = l - 1; i >= 0; i--) {
+        const uint32_t sh = (uint32_t)b.shape[i];
+        src += (size_t)(rem % sh) * b.xstride[i];
+        rem /= sh;
+    }
+    u4 v;
+    if (b.xstride[l]) {
+        v = *(const u4*)(x + src);
+    } else {
+        const uint32_t e = sizeof(T) == 2 ? (uint32_t)x[src] * 0x10001u : (uint32_t)x[src];
+        v = u4{e, e, e, e};
+    }
+    *(u4*)(y + (size_t)g * V) = v;
+}
+
+tlhip_status launch_broadcast(hipStream_t s, const void* x, void* y, int elem, const BcastDims& full) {
     int64_t total = 1;
-    for (int i = 0; i < b.nd; i++) total *= b.shape[i];
+    for (int i = 0; i < full.nd; i++) total *= full.shape[i];
     if (total <= 0) return TLHIP_OK;
+    // dims of 1 dropped, neighbours that advance together (or both repeat)
+    // merged: fewer divisions per element, longer inner rows
+    BcastDims b;
+    for (int i = 0; i < full.nd; i++) {
+        if (full.shape[i] == 1) continue;
+        if (b.nd && (full.xstride[i] ? b.xstride[b.nd - 1] == full.xstride[i] * full.shape[i] : b.xstride[b.nd - 1] == 0)) {
+            b.shape[b.nd - 1] *= full.shape[i];
+            b.xstride[b.nd - 1] = full.xstride[i];
+            continue;
+        }
+        b.shape[b.nd] = full.shape[i];
+        b.xstride[b.nd++] = full.xstride[i];
+    }
+    if (!b.nd) {
+        b.nd = 1;
+        b.shape[0] = 1;
+    }
+    const int V = 16 / elem;
+    bool wide = total >= 4096 && total / V <= 0xffffff00ll && b.shape[b.nd - 1] % V == 0 && b.xstride[b.nd - 1] <= 1 &&
+                ((uintptr_t)x | (uintptr_t)y) % 16 == 0;
+    for (int i = 0; i + 1 < b.nd; i++) wide = wide && (b.xstride[b.nd - 1] == 0 || b.xstride[i] % V == 0);
+    if (wide) {
+        const uint32_t n = (uint32_t)(total / V);
+        const dim3 grid((n + 255) / 256);
+        if (elem == 2) hipLaunchKernelGGL(broadcast16_kernel<uint16_t>, grid, dim3(256), 0, s, (const uint16_t*)x, (uint16_t*)y, n, b);
+        else hipLaunchKernelGGL(broadcast16_kernel<uint32_t>, grid, dim3(256), 0, s, (const uint32_t*)x, (uint32_t*)y, n, b);
+        return TLHIP_OK;
+    }
     const dim3 grid((unsigned)((total + 255) / 256));
     if (elem == 2) hipLaunchKernelGGL(broadcast_kernel<uint16_t>, grid, dim3(256), 0, s, (const uint16_t*)x, (uint16_t*)y, total, b);
     else hipLaunchKernelGGL(broadcast_kernel<uint32_t>, grid, dim3(256), 0, s, (const uint32_t*)x, (uint32_t*)y, total, b);

@@ -1,0 +1,93 @@
+"""The many-row forms of the TL program's builtins where they can go wrong:
+the matrix-core einsums at tile edges and odd key counts, and the 16-byte
+elementwise, mask, broadcast and one-wave-per-row softmax kernels on both
+sides of the rules that choose them."""
+import numpy as np
+import pytest
+
+from tensorlogic_amd import F32
+from tensorlogic_amd import synth as S
+from tensorlogic_amd.tensor import einsum
+
+from test_gpu_ops import assert_close, ulp_diff
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("I,J,H,Hkv,D", [(16, 16, 4, 2, 64), (15, 40, 4, 2, 64), (33, 65, 8, 2, 80), (64, 128, 4, 4, 128),
+                                         (65, 129, 6, 3, 64), (130, 31, 2, 1, 80), (31, 257, 4, 1, 128)])
+def test_einsums_many_rows(dev, oracle, I, J, H, Hkv, D):
+    q = S.normal_f16(21, f"mq{I}{D}", (I, H, D))
+    k = S.normal_f16(21, f"mk{J}{D}", (J, Hkv, D))
+    v = S.normal_f16(21, f"mv{J}{D}", (J, Hkv, D))
+    sc = einsum("ihd,jhd->ihj", dev.tensor(q), dev.tensor(k)).numpy()
+    assert_close(sc, oracle.einsum_scores(q, k), what=f"scores {I}x{J} H{H}/{Hkv} D{D}")
+    p = np.random.default_rng(I + J).random((I, H, J)).astype(np.float32)
+    p = (p / p.sum(-1, keepdims=True)).astype(np.float16)
+    out = einsum("ihj,jhd->ihd", dev.tensor(p), dev.tensor(v)).numpy()
+    assert_close(out, oracle.einsum_context(p, v), what=f"context {I}x{J} H{H}/{Hkv} D{D}")
+
+
+def test_einsums_keep_non_finite_values_apart(dev):
+    """An infinite query row, key or value shows up only where it takes part:
+    padding rows and keys of the tiles add nothing."""
+    I, J, H, D = 37, 71, 2, 64
+    q, k, v = (S.normal_f16(22, n, s) for n, s in (("q", (I, H, D)), ("k", (J, H, D)), ("v", (J, H, D))))
+    q[36, 0, 3] = np.inf
+    k[70, 1, 0] = np.nan
+    sc = einsum("ihd,jhd->ihj", dev.tensor(q), dev.tensor(k)).numpy()
+    want = np.zeros((I, H, J), bool)
+    want[36, 0] = True
+    want[:, 1, 70] = True
+    assert np.array_equal(~np.isfinite(sc), want)
+    v[70, 0, 5] = np.inf
+    p = np.full((I, H, J), 1.0 / J, np.float16)
+    out = einsum("ihj,jhd->ihd", dev.tensor(p), dev.tensor(v)).numpy()
+    assert np.array_equal(np.isposinf(out), np.broadcast_to(np.arange(D) == 5, (I, H, D)) & (np.arange(H) == 0)[None, :, None])
+
+
+@pytest.mark.parametrize("rows,n", [(70000 // 8, 8), (33, 2048), (65, 1025), (31, 2113)])
+def test_elementwise_wide(dev, oracle, rows, n):
+    x = S.normal_f16(23, f"x{n}", (rows, n), 0.0, 4.0)
+    u = S.normal_f16(23, f"u{n}", (rows, n))
+    b = S.normal_f16(23, f"b{n}", (n,))
+    tx, tu, tb = dev.tensor(x), dev.tensor(u), dev.tensor(b)
+    for got, ref in ((tx.sigmoid(), oracle.sigmoid(x)), (tx.silu(), oracle.silu(x)), (tx.gelu(), oracle.gelu(x)),
+                     (tx.silu_mul(tu), oracle.swiglu(x, u))):
+        assert ulp_diff(got.numpy(), ref).max() <= 1
+    f = np.float32
+    for got, ref in ((tx + tu, x.astype(f) + u), (tx * tu, x.astype(f) * u), (tx * 0.125, x.astype(f) * f(0.125)),
+                     (tx + tb, x.astype(f) + b), (tx * tb, x.astype(f) * b)):
+        assert np.array_equal(got.numpy().view(np.uint16), ref.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("I,H,J", [(48, 32, 48), (40, 32, 61), (130, 4, 136)])
+def test_mask_wide(dev, I, H, J):
+    sc = S.normal_f16(24, f"s{I}{J}", (I, H, J))
+    m = (np.random.default_rng(J).random((I, J)) < 0.5).astype(np.float16)
+    m[0, 0] = -0.0
+    full = np.broadcast_to(m[:, None, :], (I, H, J))
+    want = np.where(full == 0, np.float16(-10000), sc)
+    for mask in (m, np.ascontiguousarray(full)):
+        got = dev.tensor(sc).apply_attention_mask(dev.tensor(mask)).numpy()
+        assert np.array_equal(got.view(np.uint16), want.view(np.uint16))
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("src,dst", [((70, 4, 1, 64), (70, 4, 8, 64)), ((80, 1, 80), (80, 32, 80)), ((81, 1, 81), (81, 9, 81)),
+                                     ((1, 1, 1), (1, 32, 300)), ((700, 1), (700, 16)), ((1, 24), (300, 24)), ((5, 1, 3), (5, 40, 3)),
+                                     ((64, 1, 8, 1), (64, 3, 8, 16)), ((1,), (4100,))])
+def test_broadcast_wide(dev, dtype, src, dst):
+    x = np.random.default_rng(3).standard_normal(src).astype(dtype)
+    got = dev.tensor(x, F32 if dtype == np.float32 else 0).broadcast_to(dst).numpy()
+    assert np.array_equal(got, np.broadcast_to(x, dst))
+
+
+@pytest.mark.parametrize("rows,n", [(5, 1), (7, 9), (6, 64), (5, 127), (6, 130), (9, 401), (3, 512), (4, 1024), (2, 1025)])
+def test_softmax_one_wave_rows(dev, oracle, rows, n):
+    x = S.normal_f16(25, f"x{n}", (rows, n), 0.0, 3.0)
+    x[1] = -10000.0        # a fully masked row, and infinities among values
+    if n > 8:
+        x[0, n - 1], x[0, 3] = np.inf, -np.inf
+    got = dev.tensor(x).softmax().numpy()
+    assert ulp_diff(got, oracle.softmax(x)).max() <= 1
