@@ -61,6 +61,16 @@ def test_elementwise_wide(dev, oracle, rows, n):
         assert np.array_equal(got.numpy().view(np.uint16), ref.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("fn", ["gelu", "sigmoid", "silu"])
+def test_activations_over_all_f16(dev, oracle, fn):
+    x = np.arange(65536, dtype=np.uint16).view(np.float16)
+    got, ref = getattr(dev.tensor(x), fn)().numpy(), getattr(oracle, fn)(x)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    # one f16 rounding of an f32 value within a few f32 ulps of the oracle's
+    assert ulp_diff(got[ok], ref[ok]).max() <= 1
+
+
 @pytest.mark.parametrize("I,H,J", [(48, 32, 48), (40, 32, 61), (130, 4, 136)])
 def test_mask_wide(dev, I, H, J):
     sc = S.normal_f16(24, f"s{I}{J}", (I, H, J))
