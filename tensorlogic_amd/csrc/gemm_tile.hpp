@@ -3,8 +3,8 @@
 // y[M, N] = x[M, K] . W[N, K]^T, K % 32 == 0, W packed Q4_0 / Q8_0 or f16.
 // A workgroup of 8 waves owns a BM x BN output tile: WM x WN waves side by
 // side, each 32 TM x 32 TN in v_mfma_f32_32x32x16_f16 tiles, and G = 8 /
-// (WM WN) groups of them that share the tile and split each K step (one or
-// two 32-element quant blocks per wave and step).  What bounds it: the LDS
+// (WM WN) groups of them that share the tile and split each K step (a
+// 32-element quant block per wave and step).  What bounds it: the LDS
 // ports, the address unit of the direct-to-LDS loads and the matrix cores are
 // each close to full at 128 x 128, so the design spends as little as it can
 // on the first two:
@@ -19,6 +19,15 @@
 //  - The loads that refill a stage are spread over the MFMAs of the next
 //    step; issued back to back after the barrier they stalled every wave at
 //    the address unit (M = 512, [5632 x 2048] Q8_0: 23.7 -> 20.7 us).
+//  - A step's scales are few bytes of many rows, and the load that brings
+//    them costs the address unit and the memory as much as 1 KB of weights
+//    does: they come for four steps at once, and the K loop is written four
+//    steps to a round, so that nothing branches on it.  Weights out of HBM /
+//    in the caches, a load of scales per step -> now, M = 512: Q8_0 [2560 x
+//    10240] 86.5 / 62.5 -> 70.9 / 59.4 us, [7680 x 2560] 29.5 / 25.1 -> 27.5 /
+//    25.1, Q4_0 [2560 x 10240] 70.2 / 61.8 -> 63.6 / 58.0 us (the short
+//    [5632 x 2048] out of the caches went from 18.7 to 19.4, out of HBM from
+//    23.0 to 21.5).
 //  - The weights stay packed in LDS and are dequantised into registers
 //    between the MFMAs of the sub-step before (RNE_f16((q - 8) d) /
 //    RNE_f16(q d), the exact values of gguf.rs:22-112).
@@ -26,12 +35,14 @@
 //    an epilogue of 8 consecutive outputs per thread: 16-byte stores, and a
 //    few hundred instructions where one unrolled over the accumulators was
 //    7,800 (fetching them cost more than 10 us per launch).
-// Measured (MI355X, back to back over three weight copies), the 64 x 32-wave
-// kernel this replaced / now: M = 512 Q8_0 [5632 x 2048] 29.5 / 20.7 us (an
+// Measured (MI355X, back to back over three weight copies), a kernel
+// of 64 x 32 waves / this one: M = 512 Q8_0 [5632 x 2048] 29.5 / 20.7 us (an
 // f16 GEMM of the platform's library takes 23.9), [7680 x 2560] 48 / 27,
 // [2560 x 10240] 54 / 38, [2560 x 2560] 28 / 16; M = 400 Q4_0 [2048 x 2048]
 // 24 / 9.5; M = 2048 Q4_0 [2048 x 5632] 74 / 54.
 #pragma once
+
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -56,19 +67,13 @@ struct TileParams {
     uint16_t *q_out, *kc, *vc;
 };
 
-// sk_dma with a scalar byte offset added to every lane's.
-template <int SZ>
+// sk_dma<16> with a scalar byte offset added to every lane's.
 __device__ __forceinline__ void tile_dma(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t off, uint32_t soff) {
     lds = __builtin_amdgcn_readfirstlane(lds);
     soff = __builtin_amdgcn_readfirstlane(soff);
-    if constexpr (SZ == 16)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(r),
-                     "s"(soff)
-                     : "memory");
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(r),
-                     "s"(soff)
-                     : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(r),
+                 "s"(soff)
+                 : "memory");
 }
 
 constexpr uint32_t SK_OOB = 0x80000000u;   // a buffer offset past every range
@@ -103,33 +108,38 @@ __device__ __forceinline__ constexpr int tile_swz(int r) {
     return (r / per_line) & mask;
 }
 
-template <int WT, int TM, int TN, int WM, int WN, int KB>
+template <int WT, int TM, int TN, int WM, int WN>
 struct Tile {
     static constexpr int G = 8 / (WM * WN);            // K groups: waves that share an output tile
-    static constexpr int NBK = G * KB;                 // 32-element blocks of K per step
+    static constexpr int NBK = G;                      // 32-element blocks of K per step, one per group
     static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, BK = 32 * NBK;
     static constexpr int WB = WT == TLHIP_F16 ? 64 : (WT == TLHIP_Q8_0 ? 32 : 16);   // bytes of one 32-weight block
     static constexpr int AR = 64 * NBK, BR = WB * NBK; // LDS row bytes
-    static constexpr int SW = NBK / 2 + 1;             // 4-byte words that hold a row's NBK scales, even or odd start
+    // The scales come a group of 4 steps at a time, in a ring of 2 groups: a
+    // load instruction costs the address unit the same whether it brings 1 KB
+    // or a step's few scales
+    static constexpr int SG = 4;   // (the K loop spells its four steps out)
+    static constexpr int SP = (SG * NBK / 2 + 1 + 3) / 4;   // 16-byte pieces that hold a row's scales, even or odd start
+    static constexpr int SR = 16 * SP;                      // LDS row bytes
     static constexpr int A_BYTES = BM * AR, B_BYTES = BN * BR;
-    static constexpr int S_BYTES = WT == TLHIP_F16 ? 0 : BN * SW * 4;
+    static constexpr int SL = WT == TLHIP_F16 ? 0 : BN * SP / 8;   // pieces per wave and group
     static constexpr int NA = A_BYTES / 8192;          // 16-byte-per-lane loads per wave and stage
     static constexpr int BL = B_BYTES / 128;           // 16-byte pieces of B per wave
     static constexpr int NB = (BL + 63) / 64;
-    static constexpr int SL = S_BYTES / 32;            // scale words per wave
-    static constexpr int C = NA + NB + (SL ? 1 : 0);   // loads per wave and stage
+    static constexpr int C = NA + NB;                  // loads per wave and stage, without the scales
     // every load runs on all 64 lanes: lanes past a wave's part fetch the next
     // wave's first pieces (the same data to the same place), the last wave's
     // go to the padding after its region
-    static constexpr int S_AT = A_BYTES + B_BYTES + 16 * (64 * NB - BL);
-    static constexpr int STAGE = (S_AT + (SL ? S_BYTES + 4 * (64 - SL) : 0) + 15) / 16 * 16;
+    static constexpr int STAGE = A_BYTES + B_BYTES + 16 * (64 * NB - BL);
+    static constexpr int SGROUP = SL ? 16 * (8 * SL + 64 - SL) : 0;
     static constexpr int ETM = TM < 2 ? TM : 2;        // M tiles of a wave that one pass of the epilogue takes
     static constexpr int EPI = 8 * ETM * TN * 4096;    // fp32 tiles of the 8 waves in one pass
-    static constexpr int NS0 = (160 * 1024) / STAGE;
-    static constexpr int NS = NS0 < 6 ? NS0 : 6;
-    static constexpr int LDS = NS * STAGE > EPI ? NS * STAGE : EPI;
-    static_assert(A_BYTES % 8192 == 0 && B_BYTES % 128 == 0 && SL <= 64 && NBK % 2 == 0, "load shapes");
-    static_assert(NS >= 2 && (NS - 1) * C < 64, "ring");
+    static constexpr int NS0 = (160 * 1024 - 2 * SGROUP) / STAGE;
+    static constexpr int NS = NS0 < SG ? NS0 : SG;   // (the next group's scales go before its first stage)
+    static constexpr int S_AT = NS * STAGE;
+    static constexpr int LDS = S_AT + 2 * SGROUP > EPI ? S_AT + 2 * SGROUP : EPI;
+    static_assert(A_BYTES % 8192 == 0 && B_BYTES % 128 == 0 && SL <= 64 && BN * SP % 8 == 0 && NBK % 2 == 0, "load shapes");
+    static_assert(NS >= 2 && (NS - 1) * C + 2 < 64, "ring");
 };
 
 // EPI_QKV_ROPE of 8 consecutive projections n .. n + 7 (f16) of row m: the
@@ -267,9 +277,12 @@ __device__ __forceinline__ void tile_store8(const TileParams& p, int m, int n, c
     }
 }
 
-template <int WT, int TM, int TN, int WM, int WN, int KB>
+template <int V>
+using Int = std::integral_constant<int, V>;
+
+template <int WT, int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
-    using L = Tile<WT, TM, TN, WM, WN, KB>;
+    using L = Tile<WT, TM, TN, WM, WN>;
     constexpr int G = L::G, BM = L::BM, BN = L::BN, NS = L::NS;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[L::LDS];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -298,11 +311,9 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
     // rows past M / N lie past the buffers' ranges: zeros, no memory access
     const __amdgpu_buffer_rsrc_t rx = sk_rsrc(p.x + (size_t)m0 * p.K, (uint32_t)mrows * xrow);
     const __amdgpu_buffer_rsrc_t rw = sk_rsrc(p.wq + (size_t)n0 * wrow, (uint32_t)nrows * wrow);
-    // (4-byte aligned: the tile's first scale is its buffer's element 0 or 1)
-    const size_t s0 = (size_t)n0 * nbr;
-    const int sodd = (int)(s0 & 1);
-    const __amdgpu_buffer_rsrc_t rd = sk_rsrc(WT == TLHIP_F16 ? (const void*)p.wq : (const void*)(p.wd + (s0 - sodd)),
-                                              WT == TLHIP_F16 ? 0u : (uint32_t)((sodd + nrows * nbr) * 2 + 3) & ~3u);
+    // (n0 is even: 4-byte aligned)
+    const __amdgpu_buffer_rsrc_t rd = sk_rsrc(WT == TLHIP_F16 ? (const void*)p.wq : (const void*)(p.wd + (size_t)n0 * nbr),
+                                              WT == TLHIP_F16 ? 0u : (uint32_t)(nrows * nbr * 2 + 3) & ~3u);
 
     // source offset of this lane's piece of each load at step kt0
     uint32_t asrc[L::NA], bsrc[L::NB], ssrc = 0;
@@ -318,87 +329,83 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
         bsrc[u] = (uint32_t)r * wrow + 16u * c + (uint32_t)kt0 * L::BR;
     }
     if constexpr (L::SL > 0) {
-        const int P = wave * L::SL + lane, n = P / L::SW, w = P % L::SW;
-        ssrc = 4u * ((uint32_t)(sodd + n * nbr + kt0 * L::NBK) / 2u + w);
+        const int P = wave * L::SL + lane, n = P / L::SP, c = P % L::SP;
+        ssrc = 4u * ((uint32_t)(n * nbr + kt0 * L::NBK) / 2u) + 16u * c;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(gl_lds_t)smem);
 
     // Load d (of L::C) of step kt0 + step into ring slot `slot`: fixed lane
     // offsets, the step in the scalar offset.  Steps past the last go to an
     // offset outside the buffers (zeros, no memory access), so that every
-    // wait counts the same loads.  (Pieces past K in a partial last step hold
+    // wait counts the same loads; the scales of a group of steps go before its
+    // first stage.  (Pieces past K in a partial last step hold
     // whatever follows in the tile's buffer; no wave computes on those blocks.)
     auto issue = [&](int d, int step, int slot) {
         const uint32_t base = lds0 + (uint32_t)slot * L::STAGE;
         const uint32_t dead = step < nk ? 0u : SK_OOB;
         const uint32_t st = step < nk ? (uint32_t)step : 0u;
         if (d < L::NA)
-            tile_dma<16>(rx, base + 1024u * (d * 8 + wave), asrc[d < L::NA ? d : 0] | dead, st * L::AR);
-        else if (d < L::NA + L::NB)
-            tile_dma<16>(rw, base + L::A_BYTES + 16u * (wave * L::BL + 64 * (d - L::NA)),
-                         bsrc[d >= L::NA && d < L::NA + L::NB ? d - L::NA : 0] | dead, st * L::BR);
+            tile_dma(rx, base + 1024u * (d * 8 + wave), asrc[d < L::NA ? d : 0] | dead, st * L::AR);
         else
-            tile_dma<4>(rd, base + L::S_AT + 4u * L::SL * wave, ssrc | dead, st * (2u * L::NBK));
+            tile_dma(rw, base + L::A_BYTES + 16u * (wave * L::BL + 64 * (d - L::NA)),
+                         bsrc[d >= L::NA && d < L::NA + L::NB ? d - L::NA : 0] | dead, st * L::BR);
     };
 
-    // operand offsets inside a stage.  This wave's blocks of a step are
-    // g * KB ..; at MFMA sub-step t lane half hh holds 8 of a block's 32
-    // elements, A and B alike:
+    auto issue_scales = [&](int grp) {
+        if constexpr (L::SL > 0)
+            tile_dma(rd, lds0 + L::S_AT + (uint32_t)(grp & 1) * L::SGROUP + 16u * L::SL * wave,
+                         ssrc | (grp * L::SG < nk ? 0u : SK_OOB), (grp * L::SG < nk ? (uint32_t)grp : 0u) * (2u * L::SG * L::NBK));
+    };
+
+    // operand offsets inside a stage.  This wave's block of a step is g; at
+    // MFMA sub-step t lane half hh holds 8 of its 32 elements, A and B alike:
     //   f16   16 t + 8 hh ..   (16 bytes per sub-step)
     //   Q8_0  16 hh + 8 t ..   (16 bytes give both sub-steps)
     //   Q4_0  16 t + 8 hh ..   (8 bytes: low nibbles t = 0, high t = 1)
-    int aoff[KB][TM][2], boff[KB][TN][2], soff[TN];
+    int aoff[TM][2], boff[TN][2], soff[TN];
 #pragma unroll
-    for (int kb = 0; kb < KB; kb++) {
-        const int blk = g * KB + kb;
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int m = 32 * (wm * TM + i) + l32;
-                const int c = 4 * blk + (WT == TLHIP_Q8_0 ? 2 * hh + t : 2 * t + hh);
-                aoff[kb][i][t] = m * L::AR + 16 * (c ^ tile_swz<L::AR>(m));
-            }
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = 32 * (wn * TN + j) + l32;
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int c = WT == TLHIP_F16 ? 4 * blk + 2 * t + hh : (WT == TLHIP_Q8_0 ? 2 * blk + hh : blk);
-                boff[kb][j][t] = L::A_BYTES + n * L::BR + 16 * (c ^ tile_swz<L::BR>(n)) + (WT == TLHIP_Q4_0 ? 8 * hh : 0);
-            }
+        for (int t = 0; t < 2; t++) {
+            const int m = 32 * (wm * TM + i) + l32;
+            const int c = 4 * g + (WT == TLHIP_Q8_0 ? 2 * hh + t : 2 * t + hh);
+            aoff[i][t] = m * L::AR + 16 * (c ^ tile_swz<L::AR>(m));
         }
-    }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int n = 32 * (wn * TN + j) + l32;
-        soff[j] = L::S_AT + 4 * L::SW * n + 2 * (((sodd + n * nbr) & 1) + g * KB);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int c = WT == TLHIP_F16 ? 4 * g + 2 * t + hh : (WT == TLHIP_Q8_0 ? 2 * g + hh : g);
+            boff[j][t] = L::A_BYTES + n * L::BR + 16 * (c ^ tile_swz<L::BR>(n)) + (WT == TLHIP_Q4_0 ? 8 * hh : 0);
+        }
+        soff[j] = L::S_AT + L::SR * n + 2 * ((n * nbr & 1) + g);
     }
 
-    // Operands of a block in registers: activations and dequantised weights
+    // Operands of the block in registers: activations and dequantised weights
     // of both MFMA sub-steps, and the block's packed weights and scales.
     h8 oa[TM][2], ob[TN][2];
     u4 rawb[TN];
     uint32_t raws[TN];
-    auto read = [&](int slot, int kb, int t) {
+    auto read = [&](int soffs, int slot, int t) {
         const uint8_t* st = smem + slot * L::STAGE;
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             if constexpr (WT == TLHIP_F16) {
-                ob[j][t] = *(const h8*)(st + boff[kb][j][t]);
+                ob[j][t] = *(const h8*)(st + boff[j][t]);
             } else if (t == 0) {
                 if constexpr (WT == TLHIP_Q8_0) {
-                    rawb[j] = *(const u4*)(st + boff[kb][j][0]);
+                    rawb[j] = *(const u4*)(st + boff[j][0]);
                 } else {
-                    const uint2 v = *(const uint2*)(st + boff[kb][j][0]);
+                    const uint2 v = *(const uint2*)(st + boff[j][0]);
                     rawb[j][0] = v.x;
                     rawb[j][1] = v.y;
                 }
-                raws[j] = *(const uint16_t*)(st + soff[j] + 2 * kb);
+                raws[j] = *(const uint16_t*)(smem + soff[j] + soffs);
             }
         }
 #pragma unroll
-        for (int i = 0; i < TM; i++) oa[i][t] = *(const h8*)(st + aoff[kb][i][t]);
+        for (int i = 0; i < TM; i++) oa[i][t] = *(const h8*)(st + aoff[i][t]);
     };
     // piece q (two per weight tile: four weights each) of sub-step t
     auto dequant = [&](int q, int t) {
@@ -409,6 +416,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
         if (WT == TLHIP_Q8_0) q8_pairs(rawb[j][2 * t + h], dd, p01, p23);
         else if (t == 0) q4_pairs(rawb[j][h] & 0x0F0F0F0Fu, dd, p01, p23);
         else q4_pairs_hi(rawb[j][h] & 0xF0F0F0F0u, dd, p01, p23);
+        asm volatile("" : "+v"(p01), "+v"(p23));   // here, not where the MFMA wants it
         u4 v = __builtin_bit_cast(u4, ob[j][t]);
         v[2 * h] = p01;
         v[2 * h + 1] = p23;
@@ -427,12 +435,13 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
     // vector issue slots), and loads [d0, d1) of stage `step`, spread out
     // because back to back they would stall the wave at the address unit.
     constexpr int NM = TM * TN, NP = WT == TLHIP_F16 ? 0 : 2 * TN;
-    auto mma = [&](int t, bool next, int d0, int d1, int step, int dslot) {
+    auto mma = [&](int t, bool next, int d0, int d1, int step, int dslot, int grp = -1) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int e = 0; e < NM; e++) {
             const int j = e / TM, i = e % TM;
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ob[j][t], oa[i][t], acc[i][j], 0, 0, 0);
+            if (grp >= 0 && e == 0) issue_scales(grp);
 #pragma unroll
             for (int d = d0 + e * (d1 - d0) / NM; d < d0 + (e + 1) * (d1 - d0) / NM; d++) issue(d, step, dslot);
             constexpr int E0 = NM / 2 - 1;
@@ -448,47 +457,49 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileParams p) {
     // stage's first operands are read, after a barrier at which every wave
     // has read the whole stage: its slot is then refilled with the stage NS
     // steps on, over the sub-steps up to the next barrier.
-    constexpr int NU = 2 * KB;   // sub-steps between barriers
-    auto dpart = [](int u) { return u * L::C / NU; };
+    // Four steps to a round of the loop: where a group of scales is issued and
+    // read is then fixed, and nothing branches inside.
+    constexpr int D1 = L::C / 2, W = (NS - 2) * L::C;
+    issue_scales(0);
 #pragma unroll
     for (int s = 0; s < NS; s++)
 #pragma unroll
-        for (int d = 0; d < (s + 1 < NS ? L::C : dpart(1)); d++) issue(d, s, s);
-    sk_wait_vm<(NS - 2) * L::C + L::C / NU>();
+        for (int d = 0; d < (s + 1 < NS ? L::C : D1); d++) issue(d, s, s);
+    sk_wait_vm<W + D1>();
     lds_barrier();
     read(0, 0, 0);
 #pragma unroll
     for (int q = 0; q < NP; q++) dequant(q, 0);
-    int slot = 0, prev = NS - 1;
-    for (int i = 0; i + 1 < nk; i++) {
+    int slot = 0, prev = NS - 1, i = 0, sgo = 0;   // sgo: LDS offset of the group of step i
+    auto step = [&](auto wait, int ph, bool scales) {
         const int nslot = slot + 1 == NS ? 0 : slot + 1;
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            read(slot, kb, 1);
-            mma(0, true, dpart(2 * kb + 1), dpart(2 * kb + 2), i - 1 + NS, prev);
-            if (kb + 1 < KB) {
-                read(slot, kb + 1, 0);
-                mma(1, true, dpart(2 * kb + 2), dpart(2 * kb + 3), i - 1 + NS, prev);
-            } else {
-                sk_wait_vm<(NS - 2) * L::C>();   // stage i + 1 has landed (loads complete in order)
-                lds_barrier();
-                read(nslot, 0, 0);
-                mma(1, true, 0, dpart(1), i + NS, slot);
-            }
-        }
+        read(0, slot, 1);
+        mma(0, true, D1, L::C, i - 1 + NS, prev);
+        sk_wait_vm<decltype(wait)::value>();   // stage i + 1 has landed (loads complete in order)
+        lds_barrier();
+        read(ph + 1 == L::SG ? L::SGROUP - sgo : sgo + (ph + 1) * 2 * L::NBK, nslot, 0);
+        mma(1, true, 0, D1, i + NS, slot, scales ? i / L::SG + 1 : -1);
         prev = slot;
         slot = nslot;
+        i++;
+    };
+    while (i + L::SG < nk) {
+        // the scales that step 0 issues may still be under way at the waits
+        // for the stages issued before them
+        constexpr int S = L::SL ? 1 : 0;
+        step(Int<W>{}, 0, true);
+        step(Int<W + (NS > 2 ? S : 0)>{}, 1, false);
+        step(Int<W + (NS > 3 ? S : 0)>{}, 2, false);
+        step(Int<W>{}, 3, false);
+        sgo = L::SGROUP - sgo;
     }
-    // the last step: this wave's blocks inside K
-    const int last_kb = nbr - (kt0 + nk - 1) * L::NBK - g * KB;
-#pragma unroll
-    for (int kb = 0; kb < KB; kb++)
-        if (kb < last_kb) {
-            read(slot, kb, 1);
-            mma(0, true, 0, 0, 0, 0);
-            if (kb + 1 < KB) read(slot, kb + 1, 0);
-            mma(1, kb + 1 < KB, 0, 0, 0, 0);
-        }
+    for (int ph = 0, left = nk - 1 - i; ph < left; ph++) step(Int<W>{}, ph, false);
+    // the last step, if this wave's block lies inside K
+    if (g < nbr - (kt0 + nk - 1) * L::NBK) {
+        read(0, slot, 1);
+        mma(0, true, 0, 0, 0, 0);
+        mma(1, false, 0, 0, 0, 0);
+    }
     sk_wait_vm<0>();   // the ring becomes the epilogue's buffer
 
     // The waves' fp32 tiles to LDS as [group][m][n] rows (C layout of the

@@ -91,10 +91,10 @@ TilePlan tile_plan(int M, int N, int K, int wt) {
 
 template <int WT, int TM, int TN, int WM, int WN>
 static void launch_tile(hipStream_t s, TileParams& p) {
-    using L = Tile<WT, TM, TN, WM, WN, 1>;
+    using L = Tile<WT, TM, TN, WM, WN>;
     p.mT = (p.M + L::BM - 1) / L::BM;
     p.nT = (p.N + L::BN - 1) / L::BN;
-    hipLaunchKernelGGL((gemm_tile_kernel<WT, TM, TN, WM, WN, 1>), dim3((unsigned)(p.mT * p.nT * p.splits)), dim3(512), 0, s, p);
+    hipLaunchKernelGGL((gemm_tile_kernel<WT, TM, TN, WM, WN>), dim3((unsigned)(p.mT * p.nT * p.splits)), dim3(512), 0, s, p);
 }
 template <int WT>
 static void launch_shape(hipStream_t s, TileParams& p, int shape) {
