@@ -560,72 +560,38 @@ __device__ __forceinline__ float ld_agent(const float* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Dim tid of one head's result from its nc chunk partials (m_c, S_c, o_c),
-// summed in chunk order. Every chunk's three loads are in flight at once,
-// AS_B chunks at a time (indices clamped, loads unconditional); up to AS_B
-// chunks that is one round trip in all. The loads are agent-scope relaxed
+// Dim tid of one head's result from its nc <= AS_B chunk partials (m_c, S_c,
+// o_c), summed in chunk order. Every chunk's three loads are in flight at once
+// (indices clamped, loads unconditional): one round trip in all. The loads are agent-scope relaxed
 // atomics in both callers: the last arriver needs them (the partials were
 // published by other workgroups of the same launch, past this XCD's L2), and
 // for the combine kernel they keep the compiler from turning the
 // uniform-address m_c / S_c loads into scalar loads sunk into the per-chunk
 // branches, one round trip per chunk.
+constexpr int AS_B = 16;
 __device__ __forceinline__ float asplit_combine(const float* pm, const float* ps, const float* po, int D, int nc, int J) {
-    constexpr int AS_B = 16;
     float M = -INFINITY, num = 0.0f, den = 0.0f;
-    if (nc <= AS_B) {
-        float mv[AS_B], sv2[AS_B], ov[AS_B];
+    float mv[AS_B], sv2[AS_B], ov[AS_B];
 #pragma unroll
-        for (int u = 0; u < AS_B; u++) {
-            const int kk = min(u, nc - 1);
-            mv[u] = ld_agent(pm + kk);
-            sv2[u] = ld_agent(ps + kk);
-            ov[u] = ld_agent(po + (size_t)kk * D);
-        }
+    for (int u = 0; u < AS_B; u++) {
+        const int kk = min(u, nc - 1);
+        mv[u] = ld_agent(pm + kk);
+        sv2[u] = ld_agent(ps + kk);
+        ov[u] = ld_agent(po + (size_t)kk * D);
+    }
 #pragma unroll
-        for (int u = 0; u < AS_B; u++)
-            if (u < nc) M = fmaxf(M, mv[u]);
-        const bool degenerate = !isfinite(M);
+    for (int u = 0; u < AS_B; u++)
+        if (u < nc) M = fmaxf(M, mv[u]);
+    const bool degenerate = !isfinite(M);
 #pragma unroll
-        for (int u = 0; u < AS_B; u++) {
-            if (u < nc) {
-                if (degenerate) {
-                    num += ov[u];
-                } else if (isfinite(mv[u])) {
-                    const float w = expf(mv[u] - M);
-                    num += w * ov[u];
-                    den += w * sv2[u];
-                }
-            }
-        }
-    } else {
-        for (int k = 0; k < nc; k += AS_B) {
-            float mv[AS_B];
-#pragma unroll
-            for (int u = 0; u < AS_B; u++) mv[u] = ld_agent(pm + min(k + u, nc - 1));
-#pragma unroll
-            for (int u = 0; u < AS_B; u++) M = fmaxf(M, mv[u]);   // (clamped repeats change nothing)
-        }
-        const bool degenerate = !isfinite(M);
-        for (int k = 0; k < nc; k += AS_B) {
-            float mv[AS_B], sv2[AS_B], ov[AS_B];
-#pragma unroll
-            for (int u = 0; u < AS_B; u++) {
-                const int kk = min(k + u, nc - 1);
-                mv[u] = ld_agent(pm + kk);
-                sv2[u] = ld_agent(ps + kk);
-                ov[u] = ld_agent(po + (size_t)kk * D);
-            }
-#pragma unroll
-            for (int u = 0; u < AS_B; u++) {
-                if (k + u < nc) {
-                    if (degenerate) {
-                        num += ov[u];
-                    } else if (isfinite(mv[u])) {
-                        const float w = expf(mv[u] - M);
-                        num += w * ov[u];
-                        den += w * sv2[u];
-                    }
-                }
+    for (int u = 0; u < AS_B; u++) {
+        if (u < nc) {
+            if (degenerate) {
+                num += ov[u];
+            } else if (isfinite(mv[u])) {
+                const float w = expf(mv[u] - M);
+                num += w * ov[u];
+                den += w * sv2[u];
             }
         }
     }
@@ -778,6 +744,68 @@ __global__ __launch_bounds__(D) void asplit_combine_kernel(AttnArgs a, SplitBufs
     a.out[(size_t)h * D + tid] = f2h(r);   // (one query row)
 }
 
+// The same for heads of more than AS_B chunks, which on one group of D threads
+// took a round trip per AS_B chunks and as many before for M (bound by those:
+// 5.8 us for 32 chunks of head dim 64): G groups of D threads take a run of
+// chunks each, so up to G AS_B chunks are one round trip, beside which the
+// workgroup finds M.  Per call, before -> now: 32 / 4 heads
+// of 64, 4000 keys 11.5 -> 9.2 us, 12000 keys 26.9 -> 16.5; 32 heads of 80, 4000
+// keys 15.4 -> 13.1; 32 / 8 of 128, 8000 keys 32.7 -> 26.7.  (256-key chunks up to
+// 4096 keys, to have 16 chunks: 10.1 us at 4000 keys of 64.)
+template <int D, int CH>
+__global__ __launch_bounds__(512) void asplit_combine_wide_kernel(AttnArgs a, SplitBufs b) {
+    constexpr int G = 512 / D;
+    __shared__ float red[8], pn[G][D], pd[G];
+    const int h = blockIdx.x, tid = threadIdx.x;
+    const int J = asplit_keys(a, b);
+    const int nc = (J + CH - 1) / CH, per = (nc + G - 1) / G;
+    const int g = min(tid / D, G - 1), d = tid % D;   // (threads past G D repeat part of group G - 1)
+    const int k1 = min(nc, (g + 1) * per);
+    const size_t hc = (size_t)h * b.nch;
+    const float *pm = b.mx + hc, *ps = b.sum + hc, *po = b.o + hc * D + d;
+    float M = -INFINITY, num = 0.0f, den = 0.0f;
+    for (int k = tid; k < nc; k += 512) M = fmaxf(M, ld_agent(pm + k));
+    bool first = true, degenerate = false;
+    for (int k = g * per; first || k < k1; k += AS_B) {
+        float mv[AS_B], sv[AS_B], ov[AS_B];
+#pragma unroll
+        for (int u = 0; u < AS_B; u++) {
+            const int kk = min(k + u, nc - 1);
+            mv[u] = ld_agent(pm + kk);
+            sv[u] = ld_agent(ps + kk);
+            ov[u] = ld_agent(po + (size_t)kk * D);
+        }
+        if (first) {   // (every thread comes here once)
+            M = block_max1<8>(M, red);
+            degenerate = !isfinite(M);
+            first = false;
+        }
+#pragma unroll
+        for (int u = 0; u < AS_B; u++) {
+            if (k + u < k1) {
+                if (degenerate) {
+                    num += ov[u];
+                } else if (isfinite(mv[u])) {
+                    const float w = expf(mv[u] - M);
+                    num += w * ov[u];
+                    den += w * sv[u];
+                }
+            }
+        }
+    }
+    if (tid < G * D) pn[g][d] = num;
+    if (tid < G * D && d == 0) pd[g] = den;
+    __syncthreads();
+    if (tid >= D) return;
+    float n = pn[0][tid], t = pd[0];
+#pragma unroll
+    for (int k = 1; k < G; k++) {
+        n += pn[k][tid];
+        t += pd[k];
+    }
+    a.out[(size_t)h * D + tid] = f2h(degenerate ? h2f(f2h(1.0f / (float)J)) * n : n / t);   // (one query row)
+}
+
 // Decode: head dims 80 / 128 from caches of more than 512 rows (one
 // workgroup per head streams too few bytes per CU there); head dim 64 only
 // past the one-workgroup kernel's score row.
@@ -806,7 +834,8 @@ static void launch_split_d(hipStream_t s, const AttnArgs& a, const SplitBufs& b,
         }
     }
     hipLaunchKernelGGL((asplit_kernel<D, NT, false, CH>), grid, dim3(NT), 0, s, a, b);
-    hipLaunchKernelGGL((asplit_combine_kernel<D, CH>), dim3((unsigned)a.H), dim3(D), 0, s, a, b);
+    if (b.nch > AS_B) hipLaunchKernelGGL((asplit_combine_wide_kernel<D, CH>), dim3((unsigned)a.H), dim3(512), 0, s, a, b);
+    else hipLaunchKernelGGL((asplit_combine_kernel<D, CH>), dim3((unsigned)a.H), dim3(D), 0, s, a, b);
 }
 template <int NT, int CH>
 static void launch_split_kernel(hipStream_t s, const AttnArgs& a, const SplitBufs& b, dim3 grid, bool xch) {

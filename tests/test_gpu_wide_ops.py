@@ -7,7 +7,7 @@ import pytest
 
 from tensorlogic_amd import F32
 from tensorlogic_amd import synth as S
-from tensorlogic_amd.tensor import einsum
+from tensorlogic_amd.tensor import attention, einsum
 
 from test_gpu_ops import assert_close, ulp_diff
 
@@ -101,3 +101,21 @@ def test_softmax_one_wave_rows(dev, oracle, rows, n):
         x[0, n - 1], x[0, 3] = np.inf, -np.inf
     got = dev.tensor(x).softmax().numpy()
     assert ulp_diff(got, oracle.softmax(x)).max() <= 1
+
+
+@pytest.mark.parametrize("D,H,Hkv", [(64, 8, 2), (80, 4, 4), (128, 8, 2)])
+@pytest.mark.parametrize("J", [2049, 2177, 4000, 8191, 16500])
+def test_one_row_over_many_key_chunks(dev, oracle, D, H, Hkv, J):
+    """17 chunks of 128 keys and more: groups of chunks that end inside, at and
+    past the last one, and more chunks than one batch of loads."""
+    q, k, v = (S.normal_f16(29, f"{n}{D}{J}", (r, hh, D)) for n, r, hh in (("q", 1, H), ("k", J, Hkv), ("v", J, Hkv)))
+    got = attention(dev.tensor(q), dev.tensor(k), dev.tensor(v), J - 1, 1 / np.sqrt(D)).numpy()
+    assert_close(got, oracle.attention(q, k, v, J - 1, 1 / np.sqrt(D), True), what=f"one row, {J} keys of {D}")
+    if J == 2177:   # keys without a finite score in most chunks, then in all: uniform over every key
+        k[:, :, 0], q[:, :, 0] = np.inf, 1.0
+        k[-1, :, 0] = 0.0
+        got = attention(dev.tensor(q), dev.tensor(k), dev.tensor(v), J - 1, 1 / np.sqrt(D)).numpy()
+        assert_close(got, np.repeat(v[-1:], H // Hkv, axis=1), what="one finite score")
+        k[-1, :, 0] = np.inf
+        got = attention(dev.tensor(q), dev.tensor(k), dev.tensor(v), J - 1, 1 / np.sqrt(D)).numpy()
+        assert_close(got, oracle.attention(q, k, v, J - 1, 1 / np.sqrt(D), True), what="no finite score")
