@@ -6,8 +6,8 @@
 // (WM WN) groups of them that share the tile and split each K step (a
 // 32-element quant block per wave and step).  What bounds it: the LDS
 // ports, the address unit of the direct-to-LDS loads and the matrix cores are
-// each close to full at 128 x 128, so the design spends as little as it can
-// on the first two:
+// each 60 - 80 % busy in the K loop at 128 x 128, so the design spends as
+// little as it can on the first two:
 //  - The waves split K instead of a narrower tile each: an activation or
 //    weight block then enters registers WN or WM times and not 4 and 2 times
 //    (8 waves of 64 x 32 read 80 KB of LDS per 64 k at 128 x 128; two groups
@@ -39,7 +39,7 @@
 // of 64 x 32 waves / this one: M = 512 Q8_0 [5632 x 2048] 29.5 / 20.7 us (an
 // f16 GEMM of the platform's library takes 23.9), [7680 x 2560] 48 / 27,
 // [2560 x 10240] 54 / 38, [2560 x 2560] 28 / 16; M = 400 Q4_0 [2048 x 2048]
-// 24 / 9.5; M = 2048 Q4_0 [2048 x 5632] 74 / 54.
+// 24 / 9.5; M = 2048 Q4_0 [2048 x 5632] 74 / 49.
 #pragma once
 
 #include <type_traits>
