@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/tl_hip.h"
+#include "broadcast_plan.hpp"
 
 namespace tlhip {
 
@@ -305,13 +306,6 @@ struct EinsumPlan {
     const uint16_t* op[EINSUM_MAX_OPS] = {};
 };
 tlhip_status launch_einsum_general(hipStream_t s, const EinsumPlan& p, uint16_t* out, int64_t n_out, int64_t n_sum);
-// broadcast_to: target dims and, per target dim, the input stride (0 where
-// the input has size 1 or no dim)
-struct BcastDims {
-    int nd = 0;
-    int64_t shape[8] = {};
-    int64_t xstride[8] = {};
-};
 tlhip_status launch_broadcast(hipStream_t s, const void* x, void* y, int elem, const BcastDims& b);
 tlhip_status launch_rope_cs(hipStream_t s, const uint16_t* x, const uint16_t* ct, const uint16_t* st, uint16_t* y,
                             int S, int H, int D);

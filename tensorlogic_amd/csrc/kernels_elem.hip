@@ -874,39 +874,21 @@ template <typename T>
 __global__ void broadcast_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t total, BcastDims b) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= total) return;
-    int64_t rem = g, src = 0;
-    for (int i = b.nd - 1; i >= 0; i--) {
-        const int64_t c = rem % b.shape[i];
-        rem /= b.shape[i];
-        src += c * b.xstride[i];
-    }
-    y[g] = x[src];
+    y[g] = x[bcast_src(b, g)];
 }
 
 // Eight f16 (four 32-bit) elements per thread, 32-bit index arithmetic
-// ([400, 1, 400] to 32 heads: 17.2 -> 5.4 us; K rows to GQA heads 5.9 -> 3.2): the
-// innermost dim a multiple of the vector and either contiguous or repeated.
+// ([400, 1, 400] to 32 heads: 17.2 -> 5.4 us; K rows to GQA heads 5.9 -> 3.2),
+// where bcast_wide_ok allows.
 template <typename T>
 __global__ __launch_bounds__(256) void broadcast16_kernel(const T* __restrict__ x, T* __restrict__ y, uint32_t total,
                                                           BcastDims b) {
     constexpr int V = 16 / sizeof(T);
     const uint32_t g = blockIdx.x * 256u + threadIdx.x;
     if (g >= total) return;
-    const int l = b.nd - 1;
-    uint32_t rem = g;
-    size_t src = 0;
-    {
-        const uint32_t per = (uint32_t)b.shape[l] / V;
-        src = (size_t)(rem % per) * V * b.xstride[l];
-        rem /= per;
-    }
-    for (int i = l - 1; i >= 0; i--) {
-        const uint32_t sh = (uint32_t)b.shape[i];
-        src += (size_t)(rem % sh) * b.xstride[i];
-        rem /= sh;
-    }
+    const size_t src = bcast_wide_src(b, g, V);
     u4 v;
-    if (b.xstride[l]) {
+    if (b.xstride[b.nd - 1]) {
         v = *(const u4*)(x + src);
     } else {
         const uint32_t e = sizeof(T) == 2 ? (uint32_t)x[src] * 0x10001u : (uint32_t)x[src];
@@ -919,28 +901,9 @@ tlhip_status launch_broadcast(hipStream_t s, const void* x, void* y, int elem, c
     int64_t total = 1;
     for (int i = 0; i < full.nd; i++) total *= full.shape[i];
     if (total <= 0) return TLHIP_OK;
-    // dims of 1 dropped, neighbours that advance together (or both repeat)
-    // merged: fewer divisions per element, longer inner rows
-    BcastDims b;
-    for (int i = 0; i < full.nd; i++) {
-        if (full.shape[i] == 1) continue;
-        if (b.nd && (full.xstride[i] ? b.xstride[b.nd - 1] == full.xstride[i] * full.shape[i] : b.xstride[b.nd - 1] == 0)) {
-            b.shape[b.nd - 1] *= full.shape[i];
-            b.xstride[b.nd - 1] = full.xstride[i];
-            continue;
-        }
-        b.shape[b.nd] = full.shape[i];
-        b.xstride[b.nd++] = full.xstride[i];
-    }
-    if (!b.nd) {
-        b.nd = 1;
-        b.shape[0] = 1;
-    }
+    const BcastDims b = bcast_merge(full);
     const int V = 16 / elem;
-    bool wide = total >= 4096 && total / V <= 0xffffff00ll && b.shape[b.nd - 1] % V == 0 && b.xstride[b.nd - 1] <= 1 &&
-                ((uintptr_t)x | (uintptr_t)y) % 16 == 0;
-    for (int i = 0; i + 1 < b.nd; i++) wide = wide && (b.xstride[b.nd - 1] == 0 || b.xstride[i] % V == 0);
-    if (wide) {
+    if (bcast_wide_ok(b, total, V) && ((uintptr_t)x | (uintptr_t)y) % 16 == 0) {
         const uint32_t n = (uint32_t)(total / V);
         const dim3 grid((n + 255) / 256);
         if (elem == 2) hipLaunchKernelGGL(broadcast16_kernel<uint16_t>, grid, dim3(256), 0, s, (const uint16_t*)x, (uint16_t*)y, n, b);
