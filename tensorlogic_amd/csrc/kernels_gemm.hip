@@ -696,7 +696,7 @@ bool gemm_rope_ok(int M, int N, int K, int wt) {
 }
 
 // Naive fp32-accumulate GEMM for f16 weights whose K is not a multiple of 32
-// (reference unit-test shapes such as [50, 122]).
+// (reference unit-test shapes such as [50, 122]), and for K = 0 of any type.
 __global__ void gemm_naive_kernel(GemmParams p) {
     int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (int64_t)p.M * p.N) return;
@@ -742,9 +742,11 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
     if (wt != TLHIP_F16 && wt != TLHIP_Q4_0 && wt != TLHIP_Q8_0)
         return fail(TLHIP_ERR_DTYPE, "gemm: weight dtype %d takes the dequantised f16 path", (int)wt);
     if (p.M <= 0 || p.N <= 0) return TLHIP_OK;
-    if (p.K % 32 != 0) {
-        if (wt != TLHIP_F16 || epi == EPI_SWIGLU_PAIR)
-            return fail(TLHIP_ERR_INVALID_OPERATION, "gemm: K=%d not a multiple of 32", p.K);
+    // K = 0 (an empty sum: zeros, or the bias) too: the tiled kernel always
+    // computes one step of K
+    if (p.K % 32 != 0 || p.K == 0) {
+        if ((wt != TLHIP_F16 && p.K != 0) || epi == EPI_SWIGLU_PAIR)
+            return fail(TLHIP_ERR_INVALID_OPERATION, "gemm: K=%d not a positive multiple of 32", p.K);
         int64_t n = (int64_t)p.M * p.N;
         hipLaunchKernelGGL(gemm_naive_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p);
         return TLHIP_OK;

@@ -59,3 +59,17 @@ def test_gemm_tile_keeps_rows_apart(dev):
     want[5] = True
     want[:, 77] = True
     assert np.array_equal(bad, want)
+
+
+@pytest.mark.parametrize("qt", [Q4_0, Q8_0, F16])
+@pytest.mark.parametrize("M", [3, 17, 70])
+def test_empty_sum(dev, qt, M):
+    """K = 0: every output is the empty sum, or the bias."""
+    N = 50
+    b = S.normal_f16(13, "eb", (N,))
+    x = dev.tensor(np.zeros((M, 0), np.float16))
+    w = dev.tensor(np.zeros((N, 0), np.float16)) if qt == F16 else dev.quantized(np.zeros(0, np.uint8), (N, 0), qt)
+    keep = dev.tensor(np.full((M, N), np.nan, np.float16))   # (freed: the outputs' blocks are not zero to begin with)
+    del keep
+    assert not x.linear(w).numpy().any()
+    assert np.array_equal(x.linear(w, dev.tensor(b)).numpy(), np.broadcast_to(b, (M, N)))
