@@ -71,6 +71,24 @@ def test_activations_over_all_f16(dev, oracle, fn):
     assert ulp_diff(got[ok], ref[ok]).max() <= 1
 
 
+def test_activation_errors_against_64_bits(dev):
+    """sigmoid and gelu over all f16 inputs against 64-bit arithmetic, in f16
+    ulps of the result.  The bars are what expf with a full divide, and tanhf,
+    give on the device (largest and mean error; sigmoid 0.5001209 / 0.1374203,
+    gelu 1.6957698 / 0.1430744): the hardware's exp and reciprocal may not be
+    further off."""
+    x = np.arange(65536, dtype=np.uint16).view(np.float16)
+    x = x[np.isfinite(x)]
+    f = x.astype(np.float64)
+    with np.errstate(over="ignore"):
+        refs = {"sigmoid": (1 / (1 + np.exp(-f)), 0.500121, 0.13742034),
+                "gelu": (0.5 * f * (1 + np.tanh(np.sqrt(2 / np.pi) * (f + 0.044715 * f**3))), 1.695770, 0.14307442)}
+    for fn, (ref, most, mean) in refs.items():
+        got = getattr(dev.tensor(x), fn)().numpy().astype(np.float64)
+        err = np.abs(got - ref) / 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ref), 2.0**-14))) - 10)
+        assert err.max() <= most and err.mean() <= mean, (fn, err.max(), err.mean())
+
+
 @pytest.mark.parametrize("I,H,J", [(48, 32, 48), (40, 32, 61), (130, 4, 136)])
 def test_mask_wide(dev, I, H, J):
     sc = S.normal_f16(24, f"s{I}{J}", (I, H, J))
