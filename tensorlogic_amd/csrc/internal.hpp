@@ -326,8 +326,8 @@ tlhip_status launch_scores(hipStream_t s, const uint16_t* q, const uint16_t* k, 
                            int I, int J, int H, int Hkv, int D);
 tlhip_status launch_context(hipStream_t s, const uint16_t* p, const uint16_t* v, uint16_t* out,
                             int I, int J, int H, int Hkv, int D);
-// The same on the matrix cores for 16 rows or more; false (nothing launched)
-// for the shapes they do not take.
+// The same on the matrix cores; false (nothing launched) for the shapes they do
+// not take.
 bool launch_scores_mfma(hipStream_t s, const uint16_t* q, const uint16_t* k, uint16_t* sc, int I, int J, int H, int Hkv,
                         int D);
 bool launch_context_mfma(hipStream_t s, const uint16_t* p, const uint16_t* v, uint16_t* out, int I, int J, int H, int Hkv,

@@ -4,8 +4,10 @@
 //
 // Both are bound by the [I, H, J] tensor they write or read.  Measured on
 // MI355X at I = J = 400, 32 heads of 64 (10.2 MB of scores), the 8-lane
-// kernels for few rows / these: scores 152 / 11.2 us, context 45 / 10.6 us.
+// kernels / these: scores 152 / 11.2 us, context 45 / 10.6 us.  einsum_rule.hpp
+// has the sizes at which each is the faster one.
 #include "device_common.hpp"
+#include "einsum_rule.hpp"
 #include "internal.hpp"
 
 namespace tlhip {
@@ -162,12 +164,9 @@ __global__ __launch_bounds__(256) void context_mfma_kernel(const uint16_t* __res
     }
 }
 
-// From 16 query rows and 16 keys on (below that most of a tile would be
-// padding, and the 8-lane kernels take about the launch floor); rows of q, k,
-// v and out on 16-byte boundaries.
-bool mfma_rows_ok(int I, int J, int D, uintptr_t aligned) {
-    return I >= 16 && J >= 16 && (D == 64 || D == 80 || D == 128) && aligned % 16 == 0;
-}
+// Head dims the kernels are built for; rows of q, k, v and out on 16-byte
+// boundaries.
+bool mfma_rows_ok(int D, uintptr_t aligned) { return (D == 64 || D == 80 || D == 128) && aligned % 16 == 0; }
 
 }  // namespace
 
@@ -175,7 +174,7 @@ bool launch_scores_mfma(hipStream_t s, const uint16_t* q, const uint16_t* k, uin
                         int D) {
     const int nJ = (J + 127) / 128, nI = (I + 63) / 64;
     const int64_t blocks = (int64_t)nJ * nI * H;
-    if (!mfma_rows_ok(I, J, D, (uintptr_t)q | (uintptr_t)k) || blocks > 0x7fffffff) return false;
+    if (!scores_mfma_wins(I, H, J) || !mfma_rows_ok(D, (uintptr_t)q | (uintptr_t)k) || blocks > 0x7fffffff) return false;
     const dim3 grid((unsigned)blocks);
     if (D == 64) hipLaunchKernelGGL(scores_mfma_kernel<64>, grid, dim3(256), 0, s, q, k, sc, I, J, H, Hkv, nJ, nI);
     else if (D == 80) hipLaunchKernelGGL(scores_mfma_kernel<80>, grid, dim3(256), 0, s, q, k, sc, I, J, H, Hkv, nJ, nI);
@@ -187,7 +186,7 @@ bool launch_context_mfma(hipStream_t s, const uint16_t* p, const uint16_t* v, ui
                          int D) {
     const int nI = (I + 31) / 32;
     const int64_t blocks = (int64_t)nI * H;
-    if (!mfma_rows_ok(I, J, D, (uintptr_t)v | (uintptr_t)out) || blocks > 0x7fffffff) return false;
+    if (!mfma_rows_ok(D, (uintptr_t)v | (uintptr_t)out) || !context_mfma_wins(I, H, J, D) || blocks > 0x7fffffff) return false;
     const dim3 grid((unsigned)blocks);
     if (D == 64) hipLaunchKernelGGL(context_mfma_kernel<64>, grid, dim3(256), 0, s, p, v, out, I, J, H, Hkv, nI);
     else if (D == 80) hipLaunchKernelGGL(context_mfma_kernel<80>, grid, dim3(256), 0, s, p, v, out, I, J, H, Hkv, nI);

@@ -9,6 +9,7 @@ from tensorlogic_amd import F32
 from tensorlogic_amd import synth as S
 from tensorlogic_amd.tensor import attention, einsum
 
+from test_einsum_rule import einsum_rule  # noqa: F401 (fixture "rule")
 from test_gpu_ops import assert_close, ulp_diff
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +27,29 @@ def test_einsums_many_rows(dev, oracle, I, J, H, Hkv, D):
     p = (p / p.sum(-1, keepdims=True)).astype(np.float16)
     out = einsum("ihj,jhd->ihd", dev.tensor(p), dev.tensor(v)).numpy()
     assert_close(out, oracle.einsum_context(p, v), what=f"context {I}x{J} H{H}/{Hkv} D{D}")
+
+
+@pytest.mark.parametrize("I,J,H,Hkv,D", [(65, 129, 32, 8, 64), (33, 257, 64, 2, 64), (17, 1000, 32, 32, 80), (100, 16, 48, 4, 80),
+                                         (129, 31, 32, 8, 80), (48, 65, 64, 64, 128), (130, 128, 16, 2, 128), (66, 17, 60, 4, 128)])
+def test_einsums_on_the_matrix_cores(dev, oracle, rule, I, J, H, Hkv, D):
+    """The same past the sizes from which the matrix-core kernels are taken:
+    rows and keys on, one past and short of their tiles."""
+    assert rule.scores(I, H, J) and rule.context(I, H, J, D)
+    test_einsums_many_rows(dev, oracle, I, J, H, Hkv, D)
+
+
+def test_context_on_the_matrix_cores_keeps_non_finite_values_apart(dev, rule):
+    I, J, H, D = 37, 71, 64, 64
+    assert rule.scores(I, H, J) and rule.context(I, H, J, D)
+    q, k, v = (S.normal_f16(22, n, s) for n, s in (("q", (I, H, D)), ("k", (J, H, D)), ("v", (J, H, D))))
+    q[36, 0, 3], k[70, 1, 0], v[70, 0, 5] = np.inf, np.nan, np.inf
+    sc = einsum("ihd,jhd->ihj", dev.tensor(q), dev.tensor(k)).numpy()
+    want = np.zeros((I, H, J), bool)
+    want[36, 0], want[:, 1, 70] = True, True
+    assert np.array_equal(~np.isfinite(sc), want)
+    p = np.full((I, H, J), 1.0 / J, np.float16)
+    out = einsum("ihj,jhd->ihd", dev.tensor(p), dev.tensor(v)).numpy()
+    assert np.array_equal(np.isposinf(out), np.broadcast_to(np.arange(D) == 5, (I, H, D)) & (np.arange(H) == 0)[None, :, None])
 
 
 def test_einsums_keep_non_finite_values_apart(dev):
