@@ -357,6 +357,21 @@ tlhip_status tlhip_model_set_sampling(tlhip_model m, float temperature, uint64_t
  * per_launch = 1 brackets every launch with its own event pair.           */
 tlhip_status tlhip_bench_linear(tlhip_ctx ctx, tlhip_tensor x, const tlhip_tensor* w, int n_w,
                                 tlhip_tensor y, int iters, int per_launch, float* avg_us);
+/* What tlhip_linear runs for x [M, K] and an F16, Q4_0, Q8_0 or Q6_K weight
+ * [N, K] (computed on the host; no device is needed):
+ *   plan[0]     tlhip_linear_kernel
+ *   plan[1, 2]  rows and columns of a workgroup's output tile (0: none)
+ *   plan[3]     K slices, plan[4] the bytes of their partials
+ *   plan[5]     1 if a prompt pass of M rows adds RoPE and the KV-cache write
+ *               in the epilogue of this product                            */
+typedef enum {
+    TLHIP_LINEAR_GEMV = 0,     /* fused dequant-GEMV, M <= 4 */
+    TLHIP_LINEAR_SKINNY = 1,   /* matrix cores, up to 64 rows */
+    TLHIP_LINEAR_TILED = 2,    /* matrix cores, direct-to-LDS ring, split K */
+    TLHIP_LINEAR_BASIC = 3,    /* matrix cores, rows past the tiled kernel's ranges */
+    TLHIP_LINEAR_PLAIN = 4     /* one thread per output: K = 0 or K % 32 != 0 */
+} tlhip_linear_kernel;
+tlhip_status tlhip_linear_plan(int64_t M, int64_t N, int64_t K, tlhip_dtype w, int64_t plan[6]);
 /* Copies `bytes` (multiple of 16) from one of n_buf source buffers to one
  * destination `iters` times with a plain 16-byte-per-lane copy kernel, back
  * to back, and returns the mean us per copy (hipEvents): the streaming

@@ -241,6 +241,7 @@ struct TilePlan {
     double us = 0.0;       // the cost model's estimate
 };
 TilePlan tile_plan(int M, int N, int K, int wt);
+void tile_dims(int shape, int* rows, int* cols);   // output tile of TilePlan::shape
 tlhip_status launch_gemm_tile(hipStream_t s, int wt, const GemvArgs& a, int epi, int ldy, const TilePlan& pl);
 // Split-K partials (fp32) stay within GEMM_SPLIT_PARTIALS_MAX bytes: the tiled
 // GEMM's plan keeps its slices' partials to it, and the skinny GEMM (5 <= M <=
@@ -250,6 +251,15 @@ constexpr size_t GEMM_SPLIT_PARTIALS_MAX = (size_t)20 << 20;
 // bytes of split-K partials launch_gemm uses when given them as a workspace
 // (0: no split; wt < 0: the most any weight type uses)
 size_t gemm_ws_bytes(int M, int N, int K, int wt);
+// what launch_gemm runs for a shape, given that workspace
+struct GemmRoute {
+    tlhip_linear_kernel kernel = TLHIP_LINEAR_PLAIN;
+    int tile_m = 0, tile_n = 0, splits = 1;
+    size_t ws_bytes = 0;
+    bool rope = false;   // gemm_rope_ok
+};
+GemmRoute gemm_route(int M, int N, int K, int wt);
+bool gemv_ok(tlhip_dtype wt, int M, int K);   // launch_gemv takes linear() of M rows
 uint16_t f32_to_f16(float f);            // host RNE rounding (F32 GGUF tensors)
 // Rows 0..src_rows-1 of a GGUF block stream [src_rows, K] go to rows
 // dst_row0 + r * dst_step of a packed tensor of dst_rows rows (to_gguf = 1:

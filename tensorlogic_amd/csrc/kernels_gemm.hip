@@ -14,6 +14,8 @@
 // (64 x 64 x 32 tiles) covers rows too long for the tiled kernel's buffer
 // ranges, gemm_naive_kernel f16 weights whose K is no multiple of 32.  Here
 // too: linear() on f32 tensors.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "gemm_tile.hpp"
@@ -569,7 +571,6 @@ static bool gemm_skinny_ok(int M, int N, int K, int wt) {
 // nothing else fits; a split leaves each wave at least two 64-k steps.
 struct SkPlan {
     int mt = 1, nt = 2, kp = 4, mtiles = 1, splits = 1;
-    double us = 0.0;   // the model's estimate
 };
 static int sk_stage_bytes(int wt, int mt, int nt) {
     const int wrow = wt == TLHIP_F16 ? 128 : (wt == TLHIP_Q8_0 ? 64 : 32);
@@ -603,20 +604,39 @@ static SkPlan sk_plan(int M, int N, int K, int wt) {
                     }
                 }
             }
-        best.us = best_us;
         if (best_us < 1e30) break;
     }
     return best;
 }
 
-// Skinny or tiled for M <= 64, by the two cost models.  sk_plan ranks skinny
-// plans among themselves; against measured launches (154 shapes, M 5 - 64) its
-// estimate e is right for Q8_0, 1.2 e for Q4_0 and 3 + e / 2 for f16, and the
-// tiled kernel's is 1 us high for f16.  The margins are for weights that
-// come from HBM, where the skinny kernel's many small workgroups start sooner:
-// M = 46, Q4_0, in a 22-layer prompt pass, skinny / tiled: [2560 x 2048] 8.6 /
-// 10.3 us, [2048 x 2048] 7.5 / 9.8, [2048 x 5632] 10.6 / 11.9, [11264 x 2048]
-// 14.3 / 11.9.
+// Skinny or tiled for M <= 64: tile_plan's estimate against one of the skinny
+// launch, fitted to it on 2660 shapes (M 5 - 64, N 64 - 32000, K 256 - 10240, the
+// three weight types), the mean of weights in the caches and out of HBM, most
+// weight on shapes where the two are close; 5 - 7 % rms.  With 0.2 us in favour of
+// the skinny kernel the pick is 0.2 - 0.5 % slower than the better one on average
+// over 560 of them drawn from those ranges, 14 % at worst.  Skinny / tiled, us:
+// f16 [256 x 2048] M = 16 6.4 / 7.9, [64 x 5632] M = 64 7.2 / 9.5, [16945 x 256]
+// M = 39 16.9 / 6.8; Q4_0 [256 x 5632] M = 16 7.6 / 9.2, [2048 x 2048] M = 46 6.5 /
+// 7.4, [11264 x 2048] M = 46 12.9 / 10.2; Q8_0 [2560 x 10240] M = 64 31.5 / 16.2.
+static bool skinny_wins(int M, int N, int K, int wt, const SkPlan& sk, const TilePlan& tile) {
+    // us: per launch; per round of 256 workgroups, per KB of weights and of all
+    // operands (busy CUs share the caches) and per 16 x 16 tile and step of a
+    // wave; per split and 10^6 partials
+    struct Fit {
+        double launch, round, weight_kb, busy_kb, mfma, split, partials;
+    };
+    const Fit f = wt == TLHIP_F16    ? Fit{1.58, 2.23, 0.0122, 0.0108, 0.0550, 1.69, 1.80}
+                  : wt == TLHIP_Q8_0 ? Fit{1.33, 2.53, 0.0300, 0.0086, 0.0493, 1.93, 4.13}
+                                     : Fit{1.11, 2.88, 0.0526, 0.0062, 0.0460, 2.07, 3.59};
+    const double bpe = wt == TLHIP_F16 ? 2.0 : (wt == TLHIP_Q8_0 ? 34.0 / 32 : 18.0 / 32);
+    const double wgs = (double)sk.mtiles * ((N + 16 * sk.nt - 1) / (16 * sk.nt)) * sk.splits, rounds = std::ceil(wgs / 256);
+    const double kx = std::min(16 * sk.mt, M) * 2e-3 * K / sk.splits, kw = 16 * sk.nt * bpe * 1e-3 * K / sk.splits;
+    double us = f.launch + rounds * (f.round + f.weight_kb * kw + f.busy_kb * std::min(wgs / 256, 1.0) * (kx + kw) +
+                                     f.mfma * K / 64.0 / sk.splits / sk.kp * sk.mt * sk.nt);
+    if (sk.splits > 1) us += f.split + f.partials * 1e-6 * sk.splits * M * N;
+    return us < tile.us + 0.2;
+}
+
 struct GemmPlan {
     int M = -1, N = 0, K = 0, wt = 0;
     bool skinny = false;
@@ -643,8 +663,7 @@ static const GemmPlan& gemm_plan(int M, int N, int K, int wt) {
     if (tile_ok(K)) p.tile = tile_plan(M, N, K, wt);
     if (gemm_skinny_ok(M, N, K, wt)) {
         p.sk = sk_plan(M, N, K, wt);
-        const double e = p.sk.us, t = tile_ok(K) ? p.tile.us : 1e30;
-        p.skinny = wt == TLHIP_F16 ? 3.0 + 0.5 * e < t - 1.0 : (wt == TLHIP_Q8_0 ? e + 0.7 < t : 1.2 * e + 0.3 < t);
+        p.skinny = !tile_ok(K) || skinny_wins(M, N, K, wt, p.sk, p.tile);
     }
     p.ws_bytes = p.skinny ? (p.sk.splits > 1 ? (size_t)p.sk.splits * M * N * sizeof(float) : 0) : p.tile.ws_bytes;
     return p;
@@ -689,6 +708,32 @@ size_t gemm_ws_bytes(int M, int N, int K, int wt) {
         return b;
     }
     return gemm_plan(M, N, K, wt).ws_bytes;
+}
+
+GemmRoute gemm_route(int M, int N, int K, int wt) {
+    GemmRoute r;
+    if (K % 32 != 0 || K == 0) {
+        r.kernel = TLHIP_LINEAR_PLAIN;
+        return r;
+    }
+    const GemmPlan& p = gemm_plan(M, N, K, wt);
+    r.rope = gemm_rope_ok(M, N, K, wt);
+    r.ws_bytes = p.ws_bytes;
+    if (p.skinny) {
+        r.kernel = TLHIP_LINEAR_SKINNY;
+        r.tile_m = 16 * p.sk.mt;
+        r.tile_n = 16 * p.sk.nt;
+        r.splits = p.sk.splits;
+    } else if (tile_ok(K)) {
+        r.kernel = TLHIP_LINEAR_TILED;
+        tile_dims(p.tile.shape, &r.tile_m, &r.tile_n);
+        r.splits = p.tile.splits;
+    } else {
+        r.kernel = TLHIP_LINEAR_BASIC;
+        r.tile_m = GBM;
+        r.tile_n = GBN;
+    }
+    return r;
 }
 
 bool gemm_rope_ok(int M, int N, int K, int wt) {

@@ -39,31 +39,39 @@ namespace {
 // for M <= 32, never more than 3 % ahead of 64 x 32.)
 struct TileShape {
     int bm, bn, bk;
-    float fix;    // us per round of workgroups: first loads, epilogue
-    float kbus;   // KB of a stage that a step streams per us, few CUs busy
-    float load;   // slowdown per step with all 256 CUs busy
 };
-constexpr TileShape SHAPES[5] = {
-    {128, 128, 128, 5.2f, 85.0f, 0.42f}, {128, 64, 128, 1.7f, 84.0f, 0.30f}, {64, 128, 128, 3.4f, 84.0f, 0.30f},
-    {64, 64, 256, 2.25f, 84.0f, 0.30f},  {64, 32, 256, 0.95f, 84.0f, 0.30f},
-};
+constexpr TileShape SHAPES[5] = {{128, 128, 128}, {128, 64, 128}, {64, 128, 128}, {64, 64, 256}, {64, 32, 256}};
 
-double stage_kb(const TileShape& t, int wt) {
-    const int blocks = t.bk / 32, wb = wt == TLHIP_F16 ? 64 : (wt == TLHIP_Q8_0 ? 32 : 16);
-    return (t.bm * t.bk * 2.0 + (double)t.bn * wb * blocks + (wt == TLHIP_F16 ? 0.0 : t.bn * (blocks / 2 + 1) * 4.0)) / 1024.0;
-}
+// The cost of a plan in us: the launch, and per round of 256 workgroups (one
+// per CU: the ring fills the LDS) what does not depend on K (first loads,
+// epilogue) and the steps, both longer by up to the `busy` terms as the CUs in
+// use go from 64 to 256; rounds after the first cost `later` more.  A split
+// adds its second launch and its partials' traffic (per 10^6 of them).
+struct TileCost {
+    double launch, split, partials;
+    struct {
+        double fix, step, busy_step, busy_fix, later;
+    } shape[5];
+};
+constexpr TileCost COST_F16 = {3.04, 3.57, 0.536, {{3.41, 1.043, 0.151, 2.61, 0.0}, {1.99, 0.444, 0.190, 0.66, 1.29},
+                                                   {1.65, 0.542, 0.190, 1.22, 0.67}, {1.44, 0.726, 0.336, 0.0, 1.25},
+                                                   {1.48, 0.363, 0.160, 0.0, 1.36}}};
+constexpr TileCost COST_Q8 = {2.50, 3.44, 0.495, {{5.65, 0.606, 0.363, 1.28, 0.0}, {2.66, 0.519, 0.101, 1.06, 0.54},
+                                                  {2.62, 0.493, 0.138, 0.83, 0.76}, {2.51, 0.534, 0.130, 0.0, 0.87},
+                                                  {2.22, 0.308, 0.123, 0.0, 0.48}}};
+constexpr TileCost COST_Q4 = {2.39, 3.45, 0.603, {{5.72, 0.568, 0.368, 0.57, 0.0}, {3.31, 0.438, 0.133, 0.64, 0.60},
+                                                  {3.07, 0.403, 0.149, 0.60, 0.69}, {2.67, 0.453, 0.119, 0.0, 0.77},
+                                                  {2.53, 0.284, 0.093, 0.0, 0.35}}};
 
 }  // namespace
 
-// Tile shape and K slices for (M, N, K, weight type).  The model is fitted to
-// measurements of every shape and split on 114 problems (M 5 - 2048, N 64 -
-// 32000, K 256 - 10240, the three weight types): a launch costs 2.9 us, plus
-// per round of 256 workgroups (one per CU: the ring fills the LDS) its fixed
-// part and its steps, each the time its bytes stream in at; a split adds 3.1
-// us and its partials' traffic.  The pick is 0.7 % slower than the best
-// measured one on average, 17 % at worst (with the weights out of HBM: 0.9 and
-// 17 %).
+// Tile shape and K slices for (M, N, K, weight type): the cheapest plan.  The
+// costs are fitted to every shape and split of 2120 problems (M 5 - 2048, N 64 -
+// 32000, K 256 - 10240, 420 of them model shapes), the mean of weights in the
+// caches and out of HBM.  The pick is 0.5 % slower than the best measured plan on
+// average, 20 % at worst; the estimate is off by 5 (packed) to 7 % rms.
 TilePlan tile_plan(int M, int N, int K, int wt) {
+    const TileCost& cost = wt == TLHIP_F16 ? COST_F16 : (wt == TLHIP_Q8_0 ? COST_Q8 : COST_Q4);
     TilePlan best;
     double best_us = 1e30;
     for (int c = 0; c < 5; c++) {
@@ -74,10 +82,13 @@ TilePlan tile_plan(int M, int N, int K, int wt) {
             const size_t bytes = (size_t)sp * M * ((N + 7) & ~7) * sizeof(float);
             if (sp > 1 && (tiles * sp > 320 || steps / sp < 2 || bytes > GEMM_SPLIT_PARTIALS_MAX)) break;
             const int64_t wgs = tiles * sp;
-            const double busy = (double)std::min<int64_t>(wgs, 256);
-            const double step_us = stage_kb(t, wt) / t.kbus * (1.0 + t.load * std::max(0.0, busy - 64.0) / 192.0);
-            double us = 2.9 + (double)((wgs + 255) / 256) * (t.fix + (steps + sp - 1) / sp * step_us);
-            if (sp > 1) us += 3.1 + (sp * 4.0 + 2.0) * M * N / 4.3e6;
+            const int64_t full = wgs / 256, last = wgs % 256;
+            const double rounds = (double)(full + (last > 0));
+            const double busy = (double)full + (last > 64 ? (last - 64) / 192.0 : 0.0);   // summed over the rounds
+            const auto& f = cost.shape[c];
+            double us = cost.launch + rounds * f.fix + busy * f.busy_fix + (rounds - 1.0) * f.later +
+                        (steps + sp - 1) / sp * (rounds * f.step + busy * f.busy_step);
+            if (sp > 1) us += cost.split + cost.partials * 1e-6 * sp * M * N;
             if (us < best_us) {
                 best_us = us;
                 best.shape = c;
@@ -88,6 +99,11 @@ TilePlan tile_plan(int M, int N, int K, int wt) {
     }
     best.us = best_us;
     return best;
+}
+
+void tile_dims(int shape, int* rows, int* cols) {
+    *rows = SHAPES[shape].bm;
+    *cols = SHAPES[shape].bn;
 }
 
 template <int WT, int TM, int TN, int WM, int WN>

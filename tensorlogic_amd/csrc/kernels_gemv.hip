@@ -361,6 +361,15 @@ static GemvParams make_params(const GemvArgs& a, int epi) {
     return p;
 }
 
+// The 64-block passes per row launch_nb (1, 2, 3 - 4 rows) and launch_m1 are
+// built for; f16 rows beyond them take gemv_generic_kernel.
+bool gemv_ok(tlhip_dtype wt, int M, int K) {
+    if (M > 4) return false;
+    if (wt == TLHIP_F16) return true;
+    const int nb = (K / 32 + 63) / 64;
+    return K > 0 && K % (wt == TLHIP_Q6_K ? 256 : 32) == 0 && nb <= (M == 1 ? 8 : (M == 2 ? 4 : 2));
+}
+
 tlhip_status launch_gemv(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int epi) {
     const GemvParams p = make_params(a, epi);
     if (p.N <= 0 || p.M <= 0) return TLHIP_OK;

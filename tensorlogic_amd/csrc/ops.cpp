@@ -213,6 +213,26 @@ tlhip_status linear_impl(tlhip_ctx ctx, tlhip_tensor x, tlhip_tensor w, tlhip_te
 
 extern "C" {
 
+tlhip_status tlhip_linear_plan(int64_t M, int64_t N, int64_t K, tlhip_dtype w, int64_t plan[6]) try {
+    if (!plan) return fail(TLHIP_ERR_INVALID_ARGUMENT, "null plan");
+    if (M < 1 || N < 1 || K < 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX)
+        return fail(TLHIP_ERR_INVALID_DIMENSION, "linear_plan: [%lld, %lld] x [%lld, %lld]^T", (long long)M, (long long)K,
+                    (long long)N, (long long)K);
+    if (w != TLHIP_F16 && !is_quant(w)) return fail(TLHIP_ERR_DTYPE, "linear_plan: weight dtype %d", (int)w);
+    if (is_quant(w) && K % quant_group(w) != 0)
+        return fail(TLHIP_ERR_INVALID_DIMENSION, "linear_plan: K %% %d", (int)quant_group(w));
+    GemmRoute r;
+    if (gemv_ok(w, (int)M, (int)K)) r.kernel = TLHIP_LINEAR_GEMV;
+    else r = gemm_route((int)M, (int)N, (int)K, w == TLHIP_Q6_K ? TLHIP_F16 : w);
+    plan[0] = r.kernel;
+    plan[1] = r.tile_m;
+    plan[2] = r.tile_n;
+    plan[3] = r.splits;
+    plan[4] = (int64_t)r.ws_bytes;
+    plan[5] = M > 1 && w != TLHIP_Q6_K && gemm_rope_ok((int)M, (int)N, (int)K, w);
+    return TLHIP_OK;
+} TLHIP_CATCH_STATUS
+
 tlhip_status tlhip_matmul(tlhip_ctx ctx, tlhip_tensor a, tlhip_tensor b, tlhip_tensor c) try {
     TLHIP_TRY(check_ctx(ctx));
     // Tensor::matmul (matmul.rs:22-60) on TensorF16 or TensorF32 operands,
