@@ -369,7 +369,8 @@ typedef enum {
     TLHIP_LINEAR_SKINNY = 1,   /* matrix cores, up to 64 rows */
     TLHIP_LINEAR_TILED = 2,    /* matrix cores, direct-to-LDS ring, split K */
     TLHIP_LINEAR_BASIC = 3,    /* matrix cores, rows past the tiled kernel's ranges */
-    TLHIP_LINEAR_PLAIN = 4     /* one thread per output: K = 0 or K % 32 != 0 */
+    TLHIP_LINEAR_PLAIN = 4,    /* one thread per output: K = 0 or K % 32 != 0 */
+    TLHIP_LINEAR_STAGED = 5    /* matrix cores, many tiles of a short K */
 } tlhip_linear_kernel;
 tlhip_status tlhip_linear_plan(int64_t M, int64_t N, int64_t K, tlhip_dtype w, int64_t plan[6]);
 /* Copies `bytes` (multiple of 16) from one of n_buf source buffers to one

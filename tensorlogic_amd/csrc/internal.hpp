@@ -243,6 +243,9 @@ struct TilePlan {
 TilePlan tile_plan(int M, int N, int K, int wt);
 void tile_dims(int shape, int* rows, int* cols);   // output tile of TilePlan::shape
 tlhip_status launch_gemm_tile(hipStream_t s, int wt, const GemvArgs& a, int epi, int ldy, const TilePlan& pl);
+// the staged GEMM (kernels_gemm_staged.hip) and its cost in us
+double staged_us(int M, int N, int K, int wt);
+tlhip_status launch_gemm_staged(hipStream_t s, int wt, const GemvArgs& a, int epi, int ldy);
 // Split-K partials (fp32) stay within GEMM_SPLIT_PARTIALS_MAX bytes: the tiled
 // GEMM's plan keeps its slices' partials to it, and the skinny GEMM (5 <= M <=
 // 64) splits at most SK_MAX_TILES_SPLIT tiles (N <= 8192 at 64 rows) into 8

@@ -10,7 +10,8 @@
 // gemm_tile_kernel (gemm_tile.hpp, kernels_gemm_tile.hip) takes every K that
 // is a multiple of 32; gemm_skinny_kernel (below) the M <= 64 shapes where it
 // is the faster one: a ring of LDS stages per wave filled by direct
-// global->LDS loads, split over K with a fence-free exchange.  gemm_kernel
+// global->LDS loads, split over K with a fence-free exchange;
+// gemm_staged_kernel (kernels_gemm_staged.hip) many tiles of a short K.  gemm_kernel
 // (64 x 64 x 32 tiles) covers rows too long for the tiled kernel's buffer
 // ranges, gemm_naive_kernel f16 weights whose K is no multiple of 32.  Here
 // too: linear() on f32 tensors.
@@ -639,7 +640,7 @@ static bool skinny_wins(int M, int N, int K, int wt, const SkPlan& sk, const Til
 
 struct GemmPlan {
     int M = -1, N = 0, K = 0, wt = 0;
-    bool skinny = false;
+    bool skinny = false, staged = false;
     SkPlan sk;
     TilePlan tile;
     size_t ws_bytes = 0;   // split-K partials
@@ -665,7 +666,15 @@ static const GemmPlan& gemm_plan(int M, int N, int K, int wt) {
         p.sk = sk_plan(M, N, K, wt);
         p.skinny = !tile_ok(K) || skinny_wins(M, N, K, wt, p.sk, p.tile);
     }
-    p.ws_bytes = p.skinny ? (p.sk.splits > 1 ? (size_t)p.sk.splits * M * N * sizeof(float) : 0) : p.tile.ws_bytes;
+    // Staged where its estimate is 5 % below the tiled kernel's, with more tiles
+    // than CUs up to K = 1024 and with fewer up to 512 (f16, whose stages leave one
+    // workgroup per CU, 512 and 384).  Past those bounds it is faster by 4 % at most
+    // and slower by up to 45 %.  Over 380 drawn shapes that pick is 0.1 - 0.4 % off
+    // the faster kernel on average, 9 % at worst.
+    const bool many = (int64_t)((M + 127) / 128) * ((N + 127) / 128) > 256;
+    p.staged = M > 64 && K % 64 == 0 && K <= (wt == TLHIP_F16 ? (many ? 512 : 384) : (many ? 1024 : 512)) &&
+               staged_us(M, N, K, wt) < 0.95 * p.tile.us;
+    p.ws_bytes = p.staged ? 0 : p.skinny ? (p.sk.splits > 1 ? (size_t)p.sk.splits * M * N * sizeof(float) : 0) : p.tile.ws_bytes;
     return p;
 }
 
@@ -724,6 +733,9 @@ GemmRoute gemm_route(int M, int N, int K, int wt) {
         r.tile_m = 16 * p.sk.mt;
         r.tile_n = 16 * p.sk.nt;
         r.splits = p.sk.splits;
+    } else if (p.staged) {
+        r.kernel = TLHIP_LINEAR_STAGED;
+        r.tile_m = r.tile_n = 128;
     } else if (tile_ok(K)) {
         r.kernel = TLHIP_LINEAR_TILED;
         tile_dims(p.tile.shape, &r.tile_m, &r.tile_n);
@@ -812,6 +824,7 @@ tlhip_status launch_gemm(hipStream_t s, tlhip_dtype wt, const GemvArgs& a, int e
         else launch_skinny<TLHIP_F16>(s, p, pl);
         return TLHIP_OK;
     }
+    if (plan.staged && epi != EPI_QKV_ROPE) return launch_gemm_staged(s, wt, a, epi, p.ldy);
     if (tile_ok(p.K)) return launch_gemm_tile(s, wt, a, epi, p.ldy, plan.tile);
     dim3 grid((unsigned)((p.N + GBN - 1) / GBN), (unsigned)((p.M + GBM - 1) / GBM));
     if (wt == TLHIP_Q4_0) hipLaunchKernelGGL(gemm_kernel<TLHIP_Q4_0>, grid, dim3(256), 0, s, p);

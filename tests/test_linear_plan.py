@@ -9,7 +9,7 @@ import pytest
 from tensorlogic_amd import F16, F32, Q4_0, Q6_K, Q8_0
 from tensorlogic_amd import _lib as L
 
-GEMV, SKINNY, TILED, BASIC, PLAIN = range(5)
+GEMV, SKINNY, TILED, BASIC, PLAIN, STAGED = range(6)
 
 
 def plan(M, N, K, wt):
@@ -42,6 +42,17 @@ def test_tile_and_split(wt, M, N, K, tile, us, other):
     assert kernel == TILED and (rows, cols, splits) == tile
 
 
+# us of the staged and of the tiled kernel's planned launch
+@pytest.mark.parametrize("wt,M,N,K,staged,tiled", [
+    (Q4_0, 2000, 23565, 256, 68.9, 98.2), (Q4_0, 1720, 11632, 448, 41.6, 55.6), (Q8_0, 916, 14250, 320, 27.7, 38.7),
+    (Q8_0, 916, 17175, 512, 42.3, 55.1), (Q8_0, 883, 15011, 768, 44.8, 53.2), (Q4_0, 1078, 8700, 448, 22.4, 29.0),
+    (Q8_0, 1024, 9583, 2048, 85.0, 74.0), (Q4_0, 855, 4827, 3456, 67.4, 53.2), (F16, 223, 8369, 1024, 28.2, 14.2),
+    (Q8_0, 738, 5483, 4928, 88.7, 75.8), (Q4_0, 129, 10240, 256, 9.8, 7.0),
+])
+def test_many_tiles_of_a_short_k_are_staged(wt, M, N, K, staged, tiled):
+    assert plan(M, N, K, wt)[0] == (STAGED if staged < tiled else TILED)
+
+
 def test_every_plan_keeps_to_its_bounds():
     """Partials of a split within the fixed workspace of the no-allocation entry
     point, none without a split, tiles of the kernels' shapes; up to 4 rows a
@@ -56,6 +67,8 @@ def test_every_plan_keeps_to_its_bounds():
             assert kernel == GEMV or (wt != F16 and K > 4096)
         elif kernel == SKINNY:
             assert M <= 64 and K % 64 == 0 and rows in (16, 32, 48, 64) and cols in (32, 64)
+        elif kernel == STAGED:
+            assert M > 64 and K % 64 == 0 and K <= 1024 and (rows, cols, splits) == (128, 128, 1)
         else:
             assert (kernel, rows, cols) in [(TILED, a, b) for a, b in ((128, 128), (128, 64), (64, 128), (64, 64), (64, 32))]
         if kernel == TILED and splits > 1:
