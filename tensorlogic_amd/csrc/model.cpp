@@ -413,7 +413,10 @@ tlhip_status enqueue_forward(tlhip_model m, int S, int pos0, const int32_t* ids_
             if (m->arch == 0) TLHIP_TRY(launch_rms_norm(s, P(m->x), P(L.norm_w), P(m->xn), S, H, m->eps));
             else TLHIP_TRY(launch_layer_norm(s, P(m->x), P(L.norm_w), P(L.norm_b), P(m->xn), S, H, m->eps));
             if (!decode && gemm_rope_ok(S, qkv_w, H, L.qkv.w->dtype)) {
-                // qkv (+ bias) + RoPE + cache write in the GEMM's epilogue
+                // qkv (+ bias) + RoPE + cache write in the GEMM's epilogue.  Prompts of
+                // 2 - 4 rows too: 4 layers of Phi-2, 3 tokens, 376 us with the multi-row
+                // GEMV and a RoPE launch, 299 so; of the llama configuration 239 and
+                // 219, of hidden 256 - 1024 151 - 198 and 138 - 182.
                 GemvArgs a;
                 a.x = P(m->xn);
                 a.wq = L.qkv.w->data;
@@ -959,7 +962,7 @@ tlhip_status tlhip_model_load(tlhip_ctx ctx, const char* path, int arch, int max
         if (e == hipSuccess) {
             const int64_t shapes[4][2] = {{H + 2 * kvd, H}, {H, H}, {arch == 0 ? 2 * I : I, H}, {H, I}};
             size_t need = 0;
-            for (int rows = 5; rows <= (int)R; rows++)
+            for (int rows = 2; rows <= (int)R; rows++)
                 for (auto& sh : shapes) need = std::max(need, gemm_ws_bytes(rows, (int)sh[0], (int)sh[1], -1));
             if (need) {
                 e = hipMalloc(&m->ws, need);

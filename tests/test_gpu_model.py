@@ -211,6 +211,26 @@ def test_llama_prefill_split_k(dev, oracle, tmp_path):
     _compare(dev, oracle, path, 0, prompt, 4, max_ctx=256)
 
 
+@pytest.mark.parametrize("n_prompt", [2, 3, 4, 5])
+def test_short_prompts(dev, oracle, tmp_path, n_prompt):
+    """Prompts of 2 to 5 tokens: the tiled GEMM's RoPE epilogue on a tile of
+    mostly padding (from 5 rows the skinny GEMM's) beside multi-row GEMVs for
+    the other projections."""
+    path = str(tmp_path / "tiny_llama_short.gguf")
+    S.write_llama_gguf(path, seed=35, **TINY_LLAMA)
+    _compare(dev, oracle, path, 0, S.token_ids(35, "prompt", n_prompt, TINY_LLAMA["vocab"]), 4)
+    path = str(tmp_path / "tiny_phi2_short.gguf")
+    S.write_phi2_gguf(path, seed=36, **TINY_PHI2)
+    _compare(dev, oracle, path, 1, S.token_ids(36, "prompt", n_prompt, TINY_PHI2["vocab"]), 4)
+
+
+def test_prompt_with_a_short_last_chunk(dev, oracle, tmp_path):
+    # 512 rows, then 3 at positions 512..514 over a filled cache
+    path = str(tmp_path / "tiny_llama_515.gguf")
+    S.write_llama_gguf(path, seed=37, **TINY_LLAMA)
+    _compare(dev, oracle, path, 0, S.token_ids(37, "prompt", 515, TINY_LLAMA["vocab"]), 4, max_ctx=600)
+
+
 def test_long_prompt_chunked_prefill(dev, oracle, tmp_path):
     # more prompt tokens than one prefill chunk holds (512 rows)
     path = str(tmp_path / "tiny_llama_long.gguf")
