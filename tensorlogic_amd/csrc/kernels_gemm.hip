@@ -610,15 +610,16 @@ static SkPlan sk_plan(int M, int N, int K, int wt) {
     return best;
 }
 
-// Skinny or tiled for M <= 64: tile_plan's estimate against one of the skinny
-// launch, fitted to it on 2660 shapes (M 5 - 64, N 64 - 32000, K 256 - 10240, the
-// three weight types), the mean of weights in the caches and out of HBM, most
-// weight on shapes where the two are close; 5 - 7 % rms.  With 0.2 us in favour of
-// the skinny kernel the pick is 0.2 - 0.5 % slower than the better one on average
-// over 560 of them drawn from those ranges, 14 % at worst.  Skinny / tiled, us:
-// f16 [256 x 2048] M = 16 6.4 / 7.9, [64 x 5632] M = 64 7.2 / 9.5, [16945 x 256]
-// M = 39 16.9 / 6.8; Q4_0 [256 x 5632] M = 16 7.6 / 9.2, [2048 x 2048] M = 46 6.5 /
-// 7.4, [11264 x 2048] M = 46 12.9 / 10.2; Q8_0 [2560 x 10240] M = 64 31.5 / 16.2.
+// Skinny or tiled for M <= 64: tile_plan's estimate against a score of the skinny
+// launch in the same us, whose constants minimise the time lost to wrong picks
+// over 2250 measured shapes (M 5 - 64, N 64 - 32000, K 256 - 10240, the three
+// weight types; weights in the caches and out of HBM; a decoder's shapes count
+// more): 0.8 (f16), 0.5 (Q4_0) and 0.9 % (Q8_0) on average, 33 % at worst, and 2.0 /
+// 0.3 / 0.3 % over a decoder's shapes.  As an estimate of the launch it is off by
+// 7 - 14 % rms.  Skinny / tiled, us: f16 [256 x 2048] M = 16 6.4 / 7.9, [64 x 5632]
+// M = 64 7.2 / 9.5, [16945 x 256] M = 39 16.9 / 6.8; Q4_0 [256 x 5632] M = 16 7.6 /
+// 9.2, [2048 x 2048] M = 46 6.5 / 7.4, [11264 x 2048] M = 46 12.9 / 10.2; Q8_0 [2560
+// x 2560] M = 46 8.0 / 8.7, [2560 x 10240] M = 64 31.5 / 16.2.
 static bool skinny_wins(int M, int N, int K, int wt, const SkPlan& sk, const TilePlan& tile) {
     // us: per launch; per round of 256 workgroups, per KB of weights and of all
     // operands (busy CUs share the caches) and per 16 x 16 tile and step of a
@@ -626,16 +627,16 @@ static bool skinny_wins(int M, int N, int K, int wt, const SkPlan& sk, const Til
     struct Fit {
         double launch, round, weight_kb, busy_kb, mfma, split, partials;
     };
-    const Fit f = wt == TLHIP_F16    ? Fit{1.58, 2.23, 0.0122, 0.0108, 0.0550, 1.69, 1.80}
-                  : wt == TLHIP_Q8_0 ? Fit{1.33, 2.53, 0.0300, 0.0086, 0.0493, 1.93, 4.13}
-                                     : Fit{1.11, 2.88, 0.0526, 0.0062, 0.0460, 2.07, 3.59};
+    const Fit f = wt == TLHIP_F16    ? Fit{1.20, 2.48, 0.0091, 0.0120, 0.032, 2.31, 2.53}
+                  : wt == TLHIP_Q8_0 ? Fit{0.04, 3.02, 0.0233, 0.0005, 0.224, 2.18, 2.49}
+                                     : Fit{0.05, 3.27, 0.0440, 0.0022, 0.156, 2.39, 0.0};
     const double bpe = wt == TLHIP_F16 ? 2.0 : (wt == TLHIP_Q8_0 ? 34.0 / 32 : 18.0 / 32);
     const double wgs = (double)sk.mtiles * ((N + 16 * sk.nt - 1) / (16 * sk.nt)) * sk.splits, rounds = std::ceil(wgs / 256);
     const double kx = std::min(16 * sk.mt, M) * 2e-3 * K / sk.splits, kw = 16 * sk.nt * bpe * 1e-3 * K / sk.splits;
     double us = f.launch + rounds * (f.round + f.weight_kb * kw + f.busy_kb * std::min(wgs / 256, 1.0) * (kx + kw) +
                                      f.mfma * K / 64.0 / sk.splits / sk.kp * sk.mt * sk.nt);
     if (sk.splits > 1) us += f.split + f.partials * 1e-6 * sk.splits * M * N;
-    return us < tile.us + 0.2;
+    return us < tile.us;
 }
 
 struct GemmPlan {
