@@ -392,9 +392,5 @@ constexpr int kAttnMaxKeys = 65536;   // keys any attention entry point reads (l
 tlhip_status launch_copy_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, int rows,
                               int row_elems, int src_stride, int dst_stride, const int32_t* d_pos,
                               int dst_row0);
-tlhip_status launch_rope_kv(hipStream_t s, const uint16_t* qkv, int qkv_stride, int S, int H,
-                            int Hkv, int D, int layout, int rot_dims, const float* table,
-                            int pos0, const int32_t* d_pos, uint16_t* q_out, uint16_t* kcache,
-                            uint16_t* vcache);
 
 }  // namespace tlhip

@@ -67,7 +67,7 @@ struct tlhip_model_s {
     std::vector<Layer> layers;
     tlhip_kvcache kv = nullptr;
     // activations, sized for max_rows tokens per pass
-    tlhip_tensor x = nullptr, xn = nullptr, qkv = nullptr, qrot = nullptr, att = nullptr, hmid = nullptr,
+    tlhip_tensor x = nullptr, xn = nullptr, qrot = nullptr, att = nullptr, hmid = nullptr,
                  logits = nullptr;
     unsigned long long* d_amax = nullptr;   // per-workgroup greedy keys of the lm_head GEMV
     uint16_t* d_vt = nullptr;                // V transposed per KV head for matrix-core prefill attention
@@ -412,39 +412,32 @@ tlhip_status enqueue_forward(tlhip_model m, int S, int pos0, const int32_t* ids_
         } else {
             if (m->arch == 0) TLHIP_TRY(launch_rms_norm(s, P(m->x), P(L.norm_w), P(m->xn), S, H, m->eps));
             else TLHIP_TRY(launch_layer_norm(s, P(m->x), P(L.norm_w), P(L.norm_b), P(m->xn), S, H, m->eps));
-            if (!decode && gemm_rope_ok(S, qkv_w, H, L.qkv.w->dtype)) {
-                // qkv (+ bias) + RoPE + cache write in the GEMM's epilogue.  Prompts of
-                // 2 - 4 rows too: 4 layers of Phi-2, 3 tokens, 376 us with the multi-row
-                // GEMV and a RoPE launch, 299 so; of the llama configuration 239 and
-                // 219, of hidden 256 - 1024 151 - 198 and 138 - 182.
-                GemvArgs a;
-                a.x = P(m->xn);
-                a.wq = L.qkv.w->data;
-                a.wd = L.qkv.w->scales;
-                a.bias = L.qkv.b ? P(L.qkv.b) : nullptr;
-                a.y = P(m->qkv);
-                a.M = S;
-                a.N = qkv_w;
-                a.K = H;
-                a.ws = m->ws;
-                a.ws_bytes = m->ws_bytes;
-                a.tile_flags = m->ctx->d_tile_flags;
-                a.nq = H;
-                a.nk = kvd;
-                a.head_dim = D;
-                a.rot = m->rot;
-                a.layout = m->arch == 0 ? 0 : 1;
-                a.pos0 = pos0;
-                a.rope_tab = m->rope_tab;
-                a.q_out = P(m->qrot);
-                a.kc = kc;
-                a.vc = vc;
-                TLHIP_TRY(launch_gemm(s, L.qkv.w->dtype, a, EPI_QKV_ROPE));
-            } else {
-                TLHIP_TRY(linear_into(s, L.qkv, P(m->xn), S, P(m->qkv), L.qkv.b ? EPI_BIAS : EPI_STORE, nullptr, 0, m->ws, m->ws_bytes, m->ctx->d_tile_flags));
-                TLHIP_TRY(launch_rope_kv(s, P(m->qkv), qkv_w, S, NH, NKV, D, m->arch == 0 ? 0 : 2, m->rot,
-                                         m->rope_tab, decode ? 0 : pos0, d_pos, P(m->qrot), kc, vc));
-            }
+            // qkv (+ bias) + RoPE + cache write in the GEMM's epilogue.  Prompts of
+            // 2 - 4 rows too: 4 layers of Phi-2, 3 tokens, 376 us with the multi-row
+            // GEMV and a RoPE launch, 299 so; of the llama configuration 239 and
+            // 219, of hidden 256 - 1024 151 - 198 and 138 - 182.
+            GemvArgs a;
+            a.x = P(m->xn);
+            a.wq = L.qkv.w->data;
+            a.wd = L.qkv.w->scales;
+            a.bias = L.qkv.b ? P(L.qkv.b) : nullptr;
+            a.M = S;
+            a.N = qkv_w;
+            a.K = H;
+            a.ws = m->ws;
+            a.ws_bytes = m->ws_bytes;
+            a.tile_flags = m->ctx->d_tile_flags;
+            a.nq = H;
+            a.nk = kvd;
+            a.head_dim = D;
+            a.rot = m->rot;
+            a.layout = m->arch == 0 ? 0 : 1;
+            a.pos0 = pos0;
+            a.rope_tab = m->rope_tab;
+            a.q_out = P(m->qrot);
+            a.kc = kc;
+            a.vc = vc;
+            TLHIP_TRY(launch_gemm(s, L.qkv.w->dtype, a, EPI_QKV_ROPE));
         }
         AttnArgs at;
         at.q = P(m->qrot);
@@ -822,7 +815,7 @@ tlhip_status tlhip_model_free(tlhip_model m) try {
     tlhip_tensor_free(m->out_norm_b);
     free_lin(m->out);
     tlhip_kvcache_free(m->kv);
-    for (tlhip_tensor t : {m->x, m->xn, m->qkv, m->qrot, m->att, m->hmid, m->logits, m->x1, m->mlp}) tlhip_tensor_free(t);
+    for (tlhip_tensor t : {m->x, m->xn, m->qrot, m->att, m->hmid, m->logits, m->x1, m->mlp}) tlhip_tensor_free(t);
     if (m->d_amax) (void)hipFree(m->d_amax);
     if (m->d_vt) (void)hipFree(m->d_vt);
     if (m->d_asplit) (void)hipFree(m->d_asplit);
@@ -929,11 +922,10 @@ tlhip_status tlhip_model_load(tlhip_ctx ctx, const char* path, int arch, int max
         m->max_rows = std::min(max_ctx, 512);
         const int64_t R = m->max_rows;
         const int64_t wide = std::max<int64_t>(H + 2 * kvd, arch == 0 ? I : I);
-        int64_t s_x[2] = {R, H}, s_qkv[2] = {R, H + 2 * kvd}, s_h[2] = {R, std::max<int64_t>(wide, I)},
+        int64_t s_x[2] = {R, H}, s_h[2] = {R, std::max<int64_t>(wide, I)},
                 s_l[1] = {m->vocab};
         if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_x, &m->x)) != TLHIP_OK) break;
         if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_x, &m->xn)) != TLHIP_OK) break;
-        if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_qkv, &m->qkv)) != TLHIP_OK) break;
         if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_x, &m->qrot)) != TLHIP_OK) break;
         if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_x, &m->att)) != TLHIP_OK) break;
         if ((st = alloc_tensor(ctx, TLHIP_F16, 2, s_h, &m->hmid)) != TLHIP_OK) break;
