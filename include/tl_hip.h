@@ -141,8 +141,8 @@ tlhip_status tlhip_linear(tlhip_ctx ctx, tlhip_tensor x, tlhip_tensor w, tlhip_t
  * tight serving loops, harnesses that forbid hipMalloc).  The split-K
  * partials of the MFMA GEMM live in a 20 MiB device array that each GPU holds
  * from library load to process end (partials beyond it -> AllocationError;
- * the library's plans keep to it: 20 MiB is e.g. [512 x 10240] @
- * [2560 x 10240]^T in 4 slices).
+ * the library's plans keep to it: the largest are 16 MiB, e.g. [1024 x 25600]
+ * @ [1024 x 25600]^T in 4 slices).
  * Its device address is resolved by tlhip_init, or on the first call if that
  * failed (a failure is reported by this call only).  A Q6_K weight with
  * M > 4 needs a dequantised f16 copy and is refused (InvalidOperation).  All

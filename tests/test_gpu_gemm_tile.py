@@ -12,21 +12,22 @@ from tensorlogic_amd import F16, Q4_0, Q8_0
 from tensorlogic_amd import synth as S
 
 from test_gpu_ops import assert_close
+from test_linear_plan import BASIC, TILED, plan
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("qt", [Q4_0, Q8_0, F16])
 @pytest.mark.parametrize("M,N,K", [
-    (65, 130, 32),      # 64 x 32 tiles, one block of K
+    (65, 130, 32),      # one block of K
     (129, 1000, 96),    # partial step, one row past two tiles
     (70, 3001, 160),    # N odd: scalar epilogue
     (130, 2050, 2080),  # 65 blocks per row
-    (96, 4100, 1056),   # 64 x 64 tiles
-    (129, 8200, 1056),  # 64 x 128 tiles
-    (513, 4099, 288),   # 128 x 64 tiles, N odd, over 256 workgroups
-    (1025, 2049, 544),  # 128 x 128 tiles, one past each way
-    (255, 8191, 1056),  # 128 x 128 tiles, one short each way
+    (96, 4100, 1056),
+    (129, 8200, 1056),
+    (513, 4099, 288),   # N odd
+    (1025, 2049, 544),  # one past a tile each way
+    (255, 8191, 1056),  # one short each way
     (66, 61, 4128),     # K split, N not a multiple of 8
     (260, 515, 8224),   # K split with a partial last step
 ])
@@ -43,6 +44,76 @@ def test_gemm_tile(dev, oracle, qt, M, N, K):
         w, ref = dev.quantized(blocks, (N, K), qt), oracle.linear_q(x, blocks, 2 if qt == Q4_0 else 8, N, b)
     y = dev.tensor(x).linear(w, dev.tensor(b)).numpy()
     assert_close(y, ref, what=f"tiled gemm {qt} {M}x{N}x{K}")
+
+
+# a shape for every tile and weight type, with K long enough that the ring of
+# scales (two groups of four steps) wraps: 10 steps of 128 or 5 of 256, the last
+# one partial; rows and columns one past or short of a tile
+EVERY_TILE = [(qt, tile, M, N, K) for tile, shapes in {
+    (128, 128): {F16: (193, 10241, 1184), Q4_0: (193, 10241, 1184), Q8_0: (193, 10241, 1184)},
+    (128, 64): {F16: (65, 8191, 1312), Q4_0: (1793, 1032, 1184), Q8_0: (1793, 1032, 1184)},
+    (64, 128): {F16: (129, 10241, 1184), Q4_0: (65, 10241, 1184), Q8_0: (65, 10241, 1184)},
+    (64, 64): {F16: (65, 4099, 1184), Q4_0: (65, 4099, 1184), Q8_0: (65, 4099, 1184)},
+    (64, 32): {F16: (65, 2049, 1184), Q4_0: (65, 2049, 1184), Q8_0: (65, 2049, 1184)},
+}.items() for qt, (M, N, K) in shapes.items()]
+
+
+@pytest.mark.parametrize("qt,tile,M,N,K", EVERY_TILE)
+def test_every_tile(dev, oracle, qt, tile, M, N, K):
+    assert plan(M, N, K, qt)[:4] == (TILED, *tile, 1)
+    test_gemm_tile(dev, oracle, qt, M, N, K)
+
+
+@pytest.mark.parametrize("qt,M,N,K,slices", [(Q4_0, 512, 2560, 10240, 3), (Q8_0, 260, 515, 8224, 3), (Q4_0, 130, 512, 8192, 8),
+                                             (F16, 66, 2560, 10240, 6), (F16, 130, 515, 8224, 4)])
+def test_split_is_deterministic(dev, oracle, qt, M, N, K, slices):
+    """The slices of a K split are summed in slice order: repeated calls give the
+    same bits, and the oracle's result."""
+    kernel, _, _, splits, ws, _ = plan(M, N, K, qt)
+    assert (kernel, splits) == (TILED, slices) and ws > 0
+    x = S.normal_f16(15, f"dx{M}x{K}", (M, K), 0.0, 0.25)
+    if qt == F16:
+        wh = S.normal_f16(15, f"dW{N}x{K}", (N, K), 0.0, 0.02)
+        w, ref = dev.tensor(wh), oracle.linear(x, wh)
+    else:
+        blocks = (S.q4_0_blocks if qt == Q4_0 else S.q8_0_blocks)(15, f"dW{N}x{K}", N, K, 1e-4, 1e-3)
+        w, ref = dev.quantized(blocks, (N, K), qt), oracle.linear_q(x, blocks, 2 if qt == Q4_0 else 8, N)
+    tx = dev.tensor(x)
+    first = tx.linear(w).numpy()
+    for _ in range(4):
+        assert np.array_equal(tx.linear(w).numpy().view(np.uint16), first.view(np.uint16))
+    assert_close(first, ref, what=f"split {qt} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("qt", [Q4_0, Q8_0, F16])
+def test_rows_past_the_tiled_ranges(dev, qt):
+    """Rows of 2^22 + 32 elements take the basic kernel: few nonzero
+    activations, small integers times a power of two, so that every sum is
+    exact."""
+    M, N, K = 6, 70, (1 << 22) + 32
+    assert plan(M, N, K, qt)[0] == BASIC
+    rng = np.random.default_rng(16)
+    at = np.unique(np.concatenate([[0, 31, 32, K - 33, K - 32, K - 1], rng.integers(0, K, 200)]))
+    x = np.zeros((M, K), np.float16)
+    x[:, at] = rng.integers(-2, 3, (M, at.size))
+    if qt == F16:
+        cols = rng.integers(-8, 8, (N, at.size)).astype(np.float16)
+        wh = np.zeros((N, K), np.float16)
+        wh[:, at] = cols
+        w = dev.tensor(wh)
+    else:
+        size, off = (18, 8) if qt == Q4_0 else (34, 0)
+        blocks = rng.integers(0, 256, (N, K // 32, size), dtype=np.uint8)
+        blocks[:, :, :2] = np.array([0.0625], np.float16).view(np.uint8)
+        e, b = at % 32, blocks[:, at // 32]
+        if qt == Q4_0:
+            q = b[:, np.arange(at.size), 2 + e % 16] >> np.where(e < 16, 0, 4) & 15
+        else:
+            q = b[:, np.arange(at.size), 2 + e].view(np.int8)
+        cols = (q.astype(np.float32) - off) * 0.0625
+        w = dev.quantized(blocks, (N, K), qt)
+    want = x[:, at].astype(np.float64) @ cols.astype(np.float64).T
+    assert np.array_equal(dev.tensor(x).linear(w).numpy(), want.astype(np.float16))
 
 
 def test_gemm_tile_keeps_rows_apart(dev):

@@ -12,11 +12,12 @@ import os
 import numpy as np
 import pytest
 
-from tensorlogic_amd import Model
+from tensorlogic_amd import F16, Q4_0, Q8_0, Model
 from tensorlogic_amd.gguf import GGML_F16, GGML_F32, GGML_Q4_0, GGML_Q8_0
 from tensorlogic_amd import synth as S
 
 from test_gpu_ops import _log_figures, assert_close, assert_logits_close, reorder_rel_l2
+from test_linear_plan import TILED, plan
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden")
@@ -164,11 +165,11 @@ def test_tiny_phi2_greedy(dev, oracle, tmp_path):
 
 @pytest.mark.parametrize("n_prompt", [65, 200])
 def test_tiny_phi2_prefill_past_64_rows(dev, oracle, tmp_path, n_prompt):
-    """A prompt of more than 64 rows takes the tiled GEMM and the separate
-    RoPE + cache write (8 outputs per thread; partial rotary: per head of 80
-    dims 16 rotated pairs written to (i, i + 16) and 48 dims passed through),
-    and from 128 rows the matrix-core attention with one head per workgroup:
-    tokens and final logits equal the oracle's."""
+    """A prompt of more than 64 rows takes the tiled GEMM, whose epilogue adds
+    RoPE and writes the cache (partial rotary: per head of 80 dims 16 rotated
+    pairs written to (i, i + 16) and 48 dims passed through), and from 128 rows
+    the matrix-core attention with one head per workgroup: tokens and final
+    logits equal the oracle's."""
     path = str(tmp_path / "tiny_phi2_rows.gguf")
     S.write_phi2_gguf(path, seed=29, **TINY_PHI2)
     prompt = S.token_ids(29, "prompt", n_prompt, TINY_PHI2["vocab"])
@@ -199,16 +200,43 @@ def test_tiny_phi2_wide_chunk_split_attention(dev, oracle, tmp_path):
 
 def test_llama_prefill_split_k(dev, oracle, tmp_path):
     """A one-layer llama with hidden 1024 and FFN 2048: a 130-row prompt
-    runs the tiled GEMM split over K for every projection (2 or 4 slices), so
-    the split-K sums with the store, residual and SwiGLU-pair epilogues (four
-    columns per thread), then the separate RoPE + cache write (interleaved
-    pairs) and the staged matrix-core attention (16 / 4 heads); tokens and
-    final logits equal the oracle's."""
+    runs the tiled GEMM with the residual, SwiGLU-pair and interleaved RoPE
+    epilogues (unsplit: test_prefill_split_over_k has the splits) and the staged
+    matrix-core attention (16 / 4 heads); tokens and final logits equal the
+    oracle's."""
     dims = dict(n_layers=1, hidden=1024, inter=2048, n_heads=16, n_kv=4, vocab=1000)
     path = str(tmp_path / "llama_split_k.gguf")
     S.write_llama_gguf(path, seed=31, **dims)
     prompt = S.token_ids(31, "prompt", 130, dims["vocab"])
     _compare(dev, oracle, path, 0, prompt, 4, max_ctx=256)
+
+
+# (arch, weights, dims, rows, the projections [N, K] whose K is split)
+@pytest.mark.parametrize("arch,qtype,dims,rows,split", [
+    # QKV + RoPE in 3 slices and gate/up in 8
+    (0, GGML_F16, dict(hidden=4096, inter=256, n_heads=32, n_kv=4), 66, [(5120, 4096), (512, 4096)]),
+    # down + residual in 8 slices
+    (0, GGML_Q4_0, dict(hidden=256, inter=8192, n_heads=4, n_kv=2), 130, [(256, 8192)]),
+    # fc2 + bias + residual in 8 slices
+    (1, GGML_Q8_0, dict(hidden=320, inter=8192, n_heads=4, rot=32), 70, [(320, 8192)]),
+])
+def test_prefill_split_over_k(dev, oracle, tmp_path, arch, qtype, dims, rows, split):
+    """The sum of a split's slices with each epilogue of a prompt pass."""
+    wt = {GGML_F16: F16, GGML_Q4_0: Q4_0, GGML_Q8_0: Q8_0}[qtype]
+    for n, k in split:
+        assert plan(rows, n, k, wt)[0] == TILED and plan(rows, n, k, wt)[3] > 1
+    path = str(tmp_path / "split.gguf")
+    (S.write_phi2_gguf if arch else S.write_llama_gguf)(path, seed=38, qtype=qtype, n_layers=1, vocab=1000, **dims)
+    _compare(dev, oracle, path, arch, S.token_ids(38, "prompt", rows, 1000), 2, max_ctx=160)
+
+
+@pytest.mark.parametrize("rot,rows", [(20, 40), (20, 70), (28, 3), (80, 66)])
+def test_phi2_rotary_widths(dev, oracle, tmp_path, rot, rows):
+    """Rotated widths that are no multiple of 8 (the one-pair-at-a-time form of
+    the tiled GEMM's RoPE epilogue) and the whole head."""
+    path = str(tmp_path / "rot.gguf")
+    S.write_phi2_gguf(path, seed=39, n_layers=1, hidden=320, inter=640, n_heads=4, vocab=1000, rot=rot)
+    _compare(dev, oracle, path, 1, S.token_ids(39, "prompt", rows, 1000), 3, max_ctx=128)
 
 
 @pytest.mark.parametrize("n_prompt", [2, 3, 4, 5])

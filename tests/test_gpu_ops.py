@@ -243,10 +243,11 @@ def test_linear_gemm(dev, oracle, qt, M, N, K):
 @pytest.mark.parametrize("qt,M,N,K", [(Q8_0, 46, 5632, 2048), (Q4_0, 512, 2048, 5632), (F16, 33, 256, 4096),
                                       (Q4_0, 46, 2048, 5632), (F16, 12, 640, 1472)])
 def test_gemm_split_k_deterministic(dev, oracle, qt, M, N, K):
-    """Split-K GEMMs sum their fp32 slices in slice order: repeated calls
-    give identical bits (no order depends on scheduling).  The skinny
-    GEMM's split (the last workgroup of a tile to arrive adds the slices)
-    also resets its arrival counters: every repeat is correct."""
+    """GEMMs give identical bits on repeated calls (no order depends on
+    scheduling): with up to 64 rows the skinny GEMM's split, whose last
+    workgroup of a tile to arrive adds the slices and resets the arrival
+    counters, so every repeat is correct; with 512 the tiled GEMM, unsplit (its
+    splits: test_gpu_gemm_tile.test_split_is_deterministic)."""
     x = S.normal_f16(7, f"xs{M}x{K}", (M, K))
     if qt == F16:
         wh = S.normal_f16(7, f"Ws{N}x{K}", (N, K), 0.0, 0.05)

@@ -13,6 +13,7 @@ from tensorlogic_amd import _lib as L
 from tensorlogic_amd import synth as S
 
 from test_gpu_ops import assert_close
+from test_linear_plan import SKINNY, TILED, plan
 
 pytestmark = pytest.mark.gpu
 
@@ -32,16 +33,14 @@ def _linear_pair(dev, oracle, qt, M, N, K, seed):
     return y_na.numpy(), y_ref.numpy(), ref
 
 
-# (qt, M, N, K): split-K GEMMs of both kernels (M <= 64: the skinny GEMM,
-# unsplit at 176 weight-row tiles, 4 and 8 slices at 64 and 8 tiles; M > 64:
-# 2 slices), then a smaller call reusing the array, then a GEMV
+# (qt, M, N, K): both kernels, split and unsplit, then a smaller call reusing the
+# array, then a GEMV (test_linear_noalloc_splits names the splits)
 @pytest.mark.parametrize("calls", [
     [(Q8_0, 46, 5632, 2048), (Q8_0, 20, 2048, 2048)],
     [(Q4_0, 512, 2048, 2048), (Q4_0, 130, 256, 2048)],
     [(Q4_0, 64, 2048, 5632), (Q8_0, 5, 256, 2048), (Q4_0, 1, 2048, 2048)],
-    # the largest partial set the split policy picks: 80 tiles x 4 slices of
-    # 128 x 128 fp32 = 20 MiB, the whole array (Phi-2 fc2 at a 512-row
-    # prefill), then a smaller split
+    # 3 slices, 15 MiB (no plan's partials are larger than 16): Phi-2 fc2 at a
+    # 512-row prefill, then a smaller call
     [(Q4_0, 512, 2560, 10240), (Q8_0, 256, 512, 2048)],
 ])
 def test_linear_noalloc_matches_linear(dev, oracle, calls):
@@ -51,8 +50,23 @@ def test_linear_noalloc_matches_linear(dev, oracle, calls):
         assert_close(got, ref, what=f"linear_noalloc call {i} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("calls", [
+    # (qt, M, N, K, kernel, K slices): the skinny GEMM, then the tiled one, each
+    # with a smaller split after a larger
+    [(Q4_0, 38, 1981, 8704, SKINNY, 8), (Q8_0, 33, 512, 4096, SKINNY, 4), (Q8_0, 5, 256, 4096, SKINNY, 4)],
+    [(Q4_0, 512, 2560, 10240, TILED, 3), (Q4_0, 130, 512, 8192, TILED, 8), (Q8_0, 66, 61, 4128, TILED, 6)],
+])
+def test_linear_noalloc_splits(dev, oracle, calls):
+    for i, (qt, M, N, K, kernel, slices) in enumerate(calls):
+        p = plan(M, N, K, qt)
+        assert (p[0], p[3]) == (kernel, slices) and 0 < p[4] <= 16 << 20
+        got, ref_dev, ref = _linear_pair(dev, oracle, qt, M, N, K, 50 + i)
+        assert np.array_equal(got.view(np.uint16), ref_dev.view(np.uint16)), f"call {i}: {M}x{N}x{K}"
+        assert_close(got, ref, what=f"linear_noalloc split {M}x{N}x{K}")
+
+
 def test_linear_noalloc_with_bias_repeated(dev, oracle):
-    """Bias epilogue through the skinny GEMM's split (8 slices), twice in a
+    """Bias epilogue through the skinny GEMM's split (4 slices), twice in a
     row on the same tensors: the second call reads only what it wrote
     itself.  The
     activations are N(0, 0.25) so that outputs stay below 8, where the bias
