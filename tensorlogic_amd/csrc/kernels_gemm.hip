@@ -612,11 +612,11 @@ static SkPlan sk_plan(int M, int N, int K, int wt) {
 
 // Skinny or tiled for M <= 64: tile_plan's estimate against a score of the skinny
 // launch in the same us, whose constants minimise the time lost to wrong picks
-// over 2250 measured shapes (M 5 - 64, N 64 - 32000, K 256 - 10240, the three
+// over 2980 measured shapes (M 5 - 64, N 64 - 32000, K 256 - 10240, the three
 // weight types; weights in the caches and out of HBM; a decoder's shapes count
-// more): 0.8 (f16), 0.5 (Q4_0) and 0.9 % (Q8_0) on average, 33 % at worst, and 2.0 /
-// 0.3 / 0.3 % over a decoder's shapes.  As an estimate of the launch it is off by
-// 7 - 14 % rms.  Skinny / tiled, us: f16 [256 x 2048] M = 16 6.4 / 7.9, [64 x 5632]
+// more): 0.8 (f16), 0.6 (Q4_0) and 0.7 % (Q8_0) on average, 32 % at worst, and 1.9 /
+// 0.3 / 0.2 % over a decoder's shapes.  As an estimate of the launch it is off by
+// 7 - 16 % rms.  Skinny / tiled, us: f16 [256 x 2048] M = 16 6.4 / 7.9, [64 x 5632]
 // M = 64 7.2 / 9.5, [16945 x 256] M = 39 16.9 / 6.8; Q4_0 [256 x 5632] M = 16 7.6 /
 // 9.2, [2048 x 2048] M = 46 6.5 / 7.4, [11264 x 2048] M = 46 12.9 / 10.2; Q8_0 [2560
 // x 2560] M = 46 8.0 / 8.7, [2560 x 10240] M = 64 31.5 / 16.2.

@@ -46,30 +46,37 @@ constexpr TileShape SHAPES[5] = {{128, 128, 128}, {128, 64, 128}, {64, 128, 128}
 // per CU: the ring fills the LDS) what does not depend on K (first loads,
 // epilogue) and the steps, both longer by up to the `busy` terms as the CUs in
 // use go from 64 to 256; rounds after the first cost `later` more.  A split
-// adds its second launch and its partials' traffic (per 10^6 of them).
+// adds its second launch, the partials' traffic and, per slice, the two loads
+// that a thread of the sum waits for: without that term [40 x 5632] @ [2048 x
+// 5632]^T took 64 x 64 tiles in 8 slices (Q8_0, 11.4 us in the caches) and not
+// 64 x 32 in 4 (9.6 us), at as many workgroups.  `weights` is their one pass from
+// HBM, `acts` the activations once per column of tiles, which narrow tiles pay
+// more often: without it f16 [100 x 2560] @ [7680 x 2560]^T took 128 x 64 tiles
+// (15.6 us in the caches, 21.7 out of HBM) and not 64 x 64 (14.3, 17.7).  All
+// three per 10^6 elements.
 struct TileCost {
-    double launch, split, partials;
+    double launch, split, slice, partials, weights, acts;
     struct {
         double fix, step, busy_step, busy_fix, later;
     } shape[5];
 };
-constexpr TileCost COST_F16 = {3.04, 3.57, 0.536, {{3.41, 1.043, 0.151, 2.61, 0.0}, {1.99, 0.444, 0.190, 0.66, 1.29},
-                                                   {1.65, 0.542, 0.190, 1.22, 0.67}, {1.44, 0.726, 0.336, 0.0, 1.25},
-                                                   {1.48, 0.363, 0.160, 0.0, 1.36}}};
-constexpr TileCost COST_Q8 = {2.50, 3.44, 0.495, {{5.65, 0.606, 0.363, 1.28, 0.0}, {2.66, 0.519, 0.101, 1.06, 0.54},
-                                                  {2.62, 0.493, 0.138, 0.83, 0.76}, {2.51, 0.534, 0.130, 0.0, 0.87},
-                                                  {2.22, 0.308, 0.123, 0.0, 0.48}}};
-constexpr TileCost COST_Q4 = {2.39, 3.45, 0.603, {{5.72, 0.568, 0.368, 0.57, 0.0}, {3.31, 0.438, 0.133, 0.64, 0.60},
-                                                  {3.07, 0.403, 0.149, 0.60, 0.69}, {2.67, 0.453, 0.119, 0.0, 0.77},
-                                                  {2.53, 0.284, 0.093, 0.0, 0.35}}};
+constexpr TileCost COST_F16 = {2.63, 2.08, 0.257, 0.484, 0.1024, 0.0467,
+                               {{4.47, 0.921, 0.0, 1.61, 0.0}, {2.74, 0.340, 0.070, 0.0, 1.27}, {2.44, 0.375, 0.237, 0.44, 0.67},
+                                {1.77, 0.669, 0.118, 0.0, 1.19}, {1.89, 0.317, 0.0, 0.0, 1.00}}};
+constexpr TileCost COST_Q8 = {2.09, 2.09, 0.277, 0.650, 0.0274, 0.0372,
+                              {{6.20, 0.562, 0.242, 0.78, 0.03}, {3.20, 0.468, 0.0, 0.83, 0.27}, {3.12, 0.448, 0.098, 0.62, 0.53},
+                               {2.92, 0.495, 0.006, 0.0, 0.53}, {2.57, 0.305, 0.0, 0.0, 0.0}}};
+constexpr TileCost COST_Q4 = {2.29, 2.23, 0.251, 0.735, 0.0125, 0.0308,
+                              {{5.82, 0.539, 0.267, 0.51, 0.0}, {3.44, 0.413, 0.038, 0.53, 0.57}, {3.18, 0.389, 0.091, 0.54, 0.71},
+                               {2.75, 0.442, 0.011, 0.0, 0.63}, {2.58, 0.283, 0.0, 0.0, 0.18}}};
 
 }  // namespace
 
 // Tile shape and K slices for (M, N, K, weight type): the cheapest plan.  The
-// costs are fitted to every shape and split of 2120 problems (M 5 - 2048, N 64 -
-// 32000, K 256 - 10240, 420 of them model shapes), the mean of weights in the
-// caches and out of HBM.  The pick is 0.5 % slower than the best measured plan on
-// average, 20 % at worst; the estimate is off by 5 (packed) to 7 % rms.
+// costs are fitted to every shape and split of 2414 problems (M 5 - 2048, N 64 -
+// 32000, K 256 - 10240, 714 of them model shapes), the mean of weights in the
+// caches and out of HBM.  The pick is 0.2 % slower than the best measured plan on
+// average, 14 % at worst; the estimate is off by 4 (packed) to 5 % rms.
 TilePlan tile_plan(int M, int N, int K, int wt) {
     const TileCost& cost = wt == TLHIP_F16 ? COST_F16 : (wt == TLHIP_Q8_0 ? COST_Q8 : COST_Q4);
     TilePlan best;
@@ -86,9 +93,10 @@ TilePlan tile_plan(int M, int N, int K, int wt) {
             const double rounds = (double)(full + (last > 0));
             const double busy = (double)full + (last > 64 ? (last - 64) / 192.0 : 0.0);   // summed over the rounds
             const auto& f = cost.shape[c];
-            double us = cost.launch + rounds * f.fix + busy * f.busy_fix + (rounds - 1.0) * f.later +
+            double us = cost.launch + 1e-6 * K * (cost.weights * N + cost.acts * M * ((N + t.bn - 1) / t.bn)) +
+                        rounds * f.fix + busy * f.busy_fix + (rounds - 1.0) * f.later +
                         (steps + sp - 1) / sp * (rounds * f.step + busy * f.busy_step);
-            if (sp > 1) us += cost.split + cost.partials * 1e-6 * sp * M * N;
+            if (sp > 1) us += cost.split + cost.slice * sp + cost.partials * 1e-6 * sp * M * N;
             if (us < best_us) {
                 best_us = us;
                 best.shape = c;

@@ -213,7 +213,7 @@ def test_llama_prefill_split_k(dev, oracle, tmp_path):
 
 # (arch, weights, dims, rows, the projections [N, K] whose K is split)
 @pytest.mark.parametrize("arch,qtype,dims,rows,split", [
-    # QKV + RoPE in 3 slices and gate/up in 8
+    # QKV + RoPE in 3 slices and gate/up in 4
     (0, GGML_F16, dict(hidden=4096, inter=256, n_heads=32, n_kv=4), 66, [(5120, 4096), (512, 4096)]),
     # down + residual in 8 slices
     (0, GGML_Q4_0, dict(hidden=256, inter=8192, n_heads=4, n_kv=2), 130, [(256, 8192)]),

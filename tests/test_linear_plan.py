@@ -36,6 +36,7 @@ def test_up_to_64_rows_take_the_faster_kernel(wt, M, N, K, want, us, other):
     (Q8_0, 396, 466, 4288, (64, 32, 1), 10.4, 15.2), (Q4_0, 978, 292, 5760, (64, 32, 1), 12.7, 17.5),
     (Q4_0, 652, 9307, 480, (128, 128, 1), 21.8, 30.3), (Q4_0, 374, 2579, 576, (64, 64, 1), 6.7, 9.1),
     (Q4_0, 130, 15689, 384, (128, 128, 1), 11.3, 14.8), (F16, 995, 108, 8320, (64, 32, 4), 11.5, 14.9),
+    (Q8_0, 40, 2048, 5632, (64, 32, 4), 10.4, 11.9), (F16, 100, 7680, 2560, (64, 64, 1), 16.0, 18.7),
 ])
 def test_tile_and_split(wt, M, N, K, tile, us, other):
     kernel, rows, cols, splits, _, _ = plan(M, N, K, wt)

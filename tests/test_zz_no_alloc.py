@@ -54,7 +54,7 @@ def test_linear_noalloc_matches_linear(dev, oracle, calls):
     # (qt, M, N, K, kernel, K slices): the skinny GEMM, then the tiled one, each
     # with a smaller split after a larger
     [(Q4_0, 38, 1981, 8704, SKINNY, 8), (Q8_0, 33, 512, 4096, SKINNY, 4), (Q8_0, 5, 256, 4096, SKINNY, 4)],
-    [(Q4_0, 512, 2560, 10240, TILED, 3), (Q4_0, 130, 512, 8192, TILED, 8), (Q8_0, 66, 61, 4128, TILED, 6)],
+    [(Q4_0, 512, 2560, 10240, TILED, 3), (Q4_0, 130, 256, 8192, TILED, 8), (Q8_0, 66, 61, 4128, TILED, 6)],
 ])
 def test_linear_noalloc_splits(dev, oracle, calls):
     for i, (qt, M, N, K, kernel, slices) in enumerate(calls):
