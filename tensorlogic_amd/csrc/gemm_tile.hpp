@@ -23,7 +23,7 @@
 //    them costs the address unit and the memory as much as 1 KB of weights
 //    does: they come for four steps at once, and the K loop is written four
 //    steps to a round, so that nothing branches on it.  Weights out of HBM /
-//    in the caches, a load of scales per step -> now, M = 512: Q8_0 [2560 x
+//    in the caches, a load of scales per step -> now, M = 512, K not split: Q8_0 [2560 x
 //    10240] 86.5 / 62.5 -> 70.9 / 59.4 us, [7680 x 2560] 29.5 / 25.1 -> 27.5 /
 //    25.1, Q4_0 [2560 x 10240] 70.2 / 61.8 -> 63.6 / 58.0 us (the short
 //    [5632 x 2048] out of the caches went from 18.7 to 19.4, out of HBM from
@@ -37,8 +37,9 @@
 //    7,800 (fetching them cost more than 10 us per launch).
 // Measured (MI355X, back to back over three weight copies), a kernel
 // of 64 x 32 waves / this one: M = 512 Q8_0 [5632 x 2048] 29.5 / 20.7 us (an
-// f16 GEMM of the platform's library takes 23.9), [7680 x 2560] 48 / 27,
-// [2560 x 10240] 54 / 38, [2560 x 2560] 28 / 16; M = 400 Q4_0 [2048 x 2048]
+// f16 GEMM of the platform's library takes 20.1; out of HBM, over 24 copies, it
+// takes 23.9 and this one 22.8), [7680 x 2560] 48 / 27, [2560 x 10240] 54 / 38 (in
+// 4 and 3 slices of K), [2560 x 2560] 28 / 16; M = 400 Q4_0 [2048 x 2048]
 // 24 / 9.5; M = 2048 Q4_0 [2048 x 5632] 74 / 49.
 #pragma once
 
